@@ -103,7 +103,9 @@ enum pd_hint { PD_HINT_NONE = 0, PD_HINT_UNSHARED_PAGES = 1, PD_HINT_RAGGED_LENG
  * per (sequence, query head) row into numerator/stats, then a merge launch
  * that combines them into out. A call whose rows hold at most 128 KB of K and
  * V per (sequence, KV head) -- min(splits * split_tokens, table_width *
- * page_size) tokens -- is instead one whole-row launch: each workgroup
+ * page_size) tokens -- is instead one whole-row launch (without shared-prefix
+ * runs up to 256 KB where the rows come to most of the CUs, and up to 512 KB
+ * where they are about one per CU): each workgroup
  * folds a row's states in LDS and writes out itself, and numerator/stats
  * are left unwritten (they remain required arguments, the workspace of the
  * reference's plan). Results agree with the two-launch path to FP32
@@ -339,8 +341,8 @@ size_t pd_workspace_bytes(int batch, int query_heads, int head_dim, int splits);
 
 /*
  * Kernel launches pd_decode / pd_decode_ex / pd_decode_scratch make for a call
- * of these formats and shapes (any lengths, bounds and stream): 1 for a
- * whole-row launch, 2 for the partition and merge launches. Returns a status
+ * of these formats and shapes without prefix runs (any lengths, bounds and
+ * stream; pd_decode_launch_plan counts them with runs): 1 for a whole-row launch, 2 for the partition and merge launches. Returns a status
  * (the shape and format checks of pd_decode_ex) and writes *launches on
  * success. No counterpart in the reference, whose decode always launches
  * twice (decode.cu:170-194); for callers that profile or account per kernel.

@@ -946,7 +946,7 @@ int pd_decode_launch_count(int q_dtype, int kv_dtype, int batch, int query_heads
                                        nullptr, f_stand_in, batch, query_heads, kv_heads, head_dim, page_size,
                                        table_width, physical_pages, splits, split_tokens, hints, nullptr,
                                        call_reach(splits, split_tokens, table_width, page_size));
-    if (q_dtype == PD_DTYPE_F32) plan_fp32(prm, kv_heads, head_dim);
+    if (q_dtype == PD_DTYPE_F32) plan_fp32(prm, kv_heads, head_dim, device_compute_units());
     else plan_mfma(prm, kv_heads, device_compute_units(), head_dim, element_size(kv_dtype));
     *launches = prm.row_mode ? 1 : 2;
     return PD_OK;
@@ -999,7 +999,7 @@ int pd_decode_launch_plan(int q_dtype, int kv_dtype, int batch, int query_heads,
                                        nullptr, f_stand_in, batch, query_heads, kv_heads, head_dim, page_size,
                                        table_width, physical_pages, ks.splits, ks.split_tokens, hints, length_bounds,
                                        reach, prefix_runs);
-    if (q_dtype == PD_DTYPE_F32) plan_fp32(prm, kv_heads, head_dim);
+    if (q_dtype == PD_DTYPE_F32) plan_fp32(prm, kv_heads, head_dim, cus);
     else plan_mfma(prm, kv_heads, cus, head_dim, static_cast<int>(element_size(kv_dtype)));
     const Grid grid = partial_grid(prm, kv_heads);
     pd_launch_plan p{};

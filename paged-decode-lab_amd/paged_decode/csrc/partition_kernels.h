@@ -962,7 +962,7 @@ int dispatch_mfma(PartialParams& prm, int kv_heads, hipStream_t stream) {
 
 template <int D>
 int dispatch_fp32(PartialParams& prm, int kv_heads, hipStream_t stream) {
-    plan_fp32(prm, kv_heads, D);
+    plan_fp32(prm, kv_heads, D, device_compute_units());
     switch (prm.head_tile) {
         case 1: return launch_fp32<D, 1>(prm, kv_heads, stream);
         case 2: return launch_fp32<D, 2>(prm, kv_heads, stream);

@@ -27,6 +27,7 @@ namespace pd {
 constexpr int kWave = 64;
 constexpr int kQuarters = 4;     // states per partition (quarters of the partition)
 constexpr int kTileTokens = 16;  // tokens per matrix-core tile
+constexpr int kMi355xCus = 256;  // compute units of an MI355X
 
 // Compacted work lists are passed in the kernel arguments for batches of up
 // to kCompactMaxBatch sequences. A tail item covers tail_span (at least
@@ -424,8 +425,7 @@ PD_HD WaveWork row_wave_work(const PartialParams& p, int b, int heads, int wave,
 template <int ALIGN>
 PD_HD int row_speculative_page(const PartialParams& p, int wave, int waves) {
     const int capacity = p.table_width << p.page_shift;
-    const int span = static_cast<int>(lmin(static_cast<int64_t>(p.splits) * p.split_tokens, capacity));
-    const int per_full = ((span + waves - 1) / waves + ALIGN - 1) / ALIGN * ALIGN;
+    const int per_full = ((p.reach + waves - 1) / waves + ALIGN - 1) / ALIGN * ALIGN;
     return imin(wave * per_full, capacity - 1) >> p.page_shift;
 }
 
@@ -718,25 +718,47 @@ inline int mfma_lds_bytes(const PartialParams& prm, int head_dim, int elem) {
     return waves * mfma_stage_bytes(head_dim, elem) + slots * combine_slot_bytes(head_dim);
 }
 
-// Whole-row launch: a full decode call whose rows are small enough to be
-// latency-bound -- at most kRowMaxBytes of K and V per (sequence, KV head) --
-// runs one workgroup per (sequence, KV head, head tile), its waves on
-// consecutive slices of the row, folds their states in LDS with the merge's
-// max-corrected sum and writes the output rows: one launch instead of two,
-// and as many waves per row as fit (up to one 16-token group each), however
-// few partitions the row has. Larger rows keep the partition launch spread
-// over all CUs: measured on MI355X, MQA B128 L1024 (256 KB per row) as 128
-// workgroups of 16 waves took 14.5 us per call, against 13.9 us for the
-// partition launch and the merge.
+// Whole-row launch: a full decode call whose rows are small enough runs one
+// workgroup per (sequence, KV head, head tile), its waves on consecutive
+// slices of the row, folds their states in LDS with the merge's max-corrected
+// sum and writes the output rows: one launch instead of two, no states written
+// and read again, and no partition left half empty by a ragged batch. Small
+// enough (K and V bytes per row):
+//   - kRowMaxBytes: always; such calls are bound by latency. Fewer rows than
+//     CUs of more bytes keep the partition launch spread over all CUs: MQA
+//     B128 L1024 (128 rows of 256 KB) took 14.5 us per call against 13.9 us.
+//   - kRowMaxBytesFull: when the rows come to at least kRowFill of the CUs.
+//   - kRowMaxBytesRound: when, besides, they are at most one per CU, so that
+//     no CU waits for others' second row.
+// Calls that may form shared-prefix items (shared_prefixes) keep the first
+// bound: their partition launch reads a shared page once for several rows.
+// Measured on MI355X (decode call, us, graph; GQA 4, D 128, FP16; two launches
+// -> whole rows; uniform / ragged / empty-to-full lengths): 256 KB, 256 rows
+// 18.1 / 14.9 / 14.6 -> 14.9 / 13.1 / 12.4, 288 rows 22.3 / 18.5 / 17.9 -> 21.3
+// / 18.0 / 17.0, 2048 rows 101.0 / 74.0 / 63.6 -> 96.6 / 63.4 / 53.0; FP8 256
+// rows 21.3 / 21.8 / 20.9 -> 19.3 / 17.8 / 17.0; FP32 512 rows 35.6 / 30.0 ->
+// 30.6 / 26.0; MQA D 64 512 rows 32.6 -> 29.5. 512 KB, 256 rows 29.4 / 23.3 /
+// 22.2 -> 26.1 / 21.2 / 19.7, but 320 rows 37.0 / 29.3 / 27.0 -> 40.1 / 30.4 /
+// 27.5 and FP8 1024 rows 110.6 -> 116.2; 1 MB, 1024 rows 131 -> 137 (ragged).
 constexpr int64_t kRowMaxBytes = 128 * 1024;
+constexpr int64_t kRowMaxBytesFull = 256 * 1024;
+constexpr int64_t kRowMaxBytesRound = 512 * 1024;
+constexpr int kRowFill = 7;  // eighths of the CUs
 constexpr int kRowWaveTokens = 16;
 
-// Whether a call's rows -- min(splits * split_tokens, table capacity) tokens
-// of K and V per (sequence, KV head), elem bytes per element -- are small
-// enough for a whole-row launch.
-inline bool rows_fit_one_launch(int64_t splits, int64_t split_tokens, int64_t capacity, int head_dim, int elem) {
-    const int64_t span = lmin(splits * split_tokens, capacity);
-    return span * head_dim * elem * 2 <= kRowMaxBytes;
+// Whether a call's rows -- `rows` of `reach` tokens (PartialParams::reach) of K
+// and V each, elem bytes per element -- are small enough for a whole-row launch.
+inline bool rows_fit_one_launch(int64_t rows, int64_t reach, int head_dim, int elem, int cus, bool shared_prefixes) {
+    const int64_t bytes = reach * head_dim * elem * 2;
+    if (bytes <= kRowMaxBytes) return true;
+    if (shared_prefixes || rows * 8 < static_cast<int64_t>(cus) * kRowFill) return false;
+    return bytes <= kRowMaxBytesFull || (bytes <= kRowMaxBytesRound && rows <= cus);
+}
+
+// Whether a call's runs and bounds let it form shared-prefix items at all
+// (group_prefixes).
+inline bool may_share_prefixes(const int32_t* runs, const int32_t* bounds, int batch, int slots) {
+    return runs != nullptr && bounds != nullptr && batch <= kCompactMaxBatch && slots >= 2;
 }
 
 // The grouping itself, as plain host arithmetic on the runs and bounds (so
@@ -761,7 +783,7 @@ inline void group_prefixes(PrefixGrouping& g, const int32_t* runs, const int32_t
         g.skip[b] = 0;
         g.order[b] = 0;
     }
-    if (runs == nullptr || bounds == nullptr || batch > kCompactMaxBatch || slots < 2) return;
+    if (!may_share_prefixes(runs, bounds, batch, slots)) return;
     int lead[kCompactMaxBatch];
     for (int b = 0; b < batch; ++b) {
         const int leader = runs[2 * b];
@@ -965,16 +987,16 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
 }
 
 // The partitions of a full decode call's two launches: coarse_split's for a
-// matrix-core call (16-bit q) that is not a whole-row launch, else the
+// matrix-core call (16-bit q) of rows above kRowMaxBytes (larger rows that run
+// as a whole-row launch have no use for the split), else the
 // caller's. kv_elem: bytes per stored K/V element; prefix_runs: the call's
 // shared-prefix runs, or nullptr.
 inline KernelSplit full_call_split(bool fp32, int kv_elem, int batch, int query_heads, int kv_heads, int head_dim,
                                    int page_size, int table_width, int splits, int split_tokens,
                                    const int32_t* length_bounds, int cus, const int32_t* prefix_runs = nullptr) {
     const KernelSplit same{splits, split_tokens};
-    if (fp32 || rows_fit_one_launch(splits, split_tokens, static_cast<int64_t>(table_width) * page_size, head_dim,
-                                    kv_elem))
-        return same;
+    const int64_t reach = lmin(static_cast<int64_t>(splits) * split_tokens, static_cast<int64_t>(table_width) * page_size);
+    if (fp32 || reach * head_dim * kv_elem * 2 <= kRowMaxBytes) return same;
     const int group = query_heads / kv_heads;
     const int gt = head_tile(group, 16);
     return coarse_split(batch, kv_heads, (group + gt - 1) / gt, head_dim, kv_elem, page_size, table_width, splits,
@@ -990,15 +1012,50 @@ constexpr int row_slot_bytes_fp32(int head_dim) { return (2 * 8 + 8 * head_dim) 
 // the 128 VGPRs of a 1024-lane workgroup without spilling: 8.
 constexpr int fp32_row_max_waves(int gt) { return gt >= 8 ? 8 : kRowMaxWaves; }
 
+// Waves of a whole-row workgroup for `rows` workgroups of `row_bytes` of K and V
+// and `outputs` output elements each, at most max_waves. A workgroup's life is
+// a chain (page ids, K and V, fold, store) that only other workgroups of its
+// CU can cover, and each wave brings 4 to 13 KB of LDS:
+//   - Rows that fit the CUs at once take 8 waves, or one lane per output
+//     element where that is more (a fold in one pass): 16-wave workgroups cost
+//     more to start and to fold than their shorter slices save.
+//   - From one row per CU on, 4 waves, so that several workgroups share a CU.
+//   - From four rows per CU on, waves of at least kRowWaveBytes each, but two
+//     of them up to eight rows per CU: the other rows fill the CU.
+// Measured on MI355X (decode call, us, graph; GQA 4, D 128, FP16; as many waves
+// as the LDS holds, up to 12 -> this rule): 2048 rows of up to 256 tokens,
+// ragged, 60.1 -> 36.4 (4 waves; 2: 36.5, 1: 37.6, 8: 54.9), 1024 rows 31.9 ->
+// 22.8, 512 rows 17.4 -> 13.2; 2048 rows of 64 tokens 18.9 -> 14.7 (1 wave;
+// 2: 16.7), of 32 tokens 14.1 -> 11.1; 1024 rows of 64 tokens 12.3 -> 9.9 (2
+// waves; 1: 11.3); 256 rows of 256 tokens 9.31 -> 8.80 (8 waves; 4: 9.38),
+// 16 rows 7.88 -> 7.34; FP8 rows of 512 tokens, 1024 rows 42.9 -> 28.6, 256
+// rows 12.4 -> 11.2. MQA rows (16 heads of 64 dims) keep 16 waves: 32 rows of
+// 512 tokens 9.45, 8 waves 9.72.
+constexpr int64_t kRowWaveBytes = 32 * 1024;
+constexpr int kRowWavesFew = 8;
+constexpr int kRowWavesMany = 4;
+
+inline int row_waves_for(int64_t rows, int64_t row_bytes, int outputs, int max_waves, int cus) {
+    if (rows <= cus) return imin(max_waves, imax(kRowWavesFew, (outputs + kWave - 1) / kWave));
+    int waves = imin(max_waves, kRowWavesMany);
+    if (rows >= 4ll * cus)
+        waves = static_cast<int>(lmin(waves, imax(rows >= 8ll * cus ? 1 : 2, static_cast<int>(row_bytes / kRowWaveBytes))));
+    return waves;
+}
+
 // Sets up a whole-row launch if the call allows it and its rows qualify;
-// slot_bytes and stage_bytes are the kernel's LDS per wave.
-inline void plan_rows(PartialParams& prm, int head_dim, int elem, int slot_bytes, int stage_bytes,
-                      int max_waves = kRowMaxWaves) {
+// slot_bytes and stage_bytes are the kernel's LDS per wave, slots the members
+// of a shared-prefix item (1: the kernel forms none).
+inline void plan_rows(PartialParams& prm, int kv_heads, int head_dim, int elem, int slot_bytes, int stage_bytes,
+                      int cus, int slots, int max_waves = kRowMaxWaves) {
     prm.row_mode = 0;
     if (!prm.row_allowed) return;
-    const int64_t capacity = static_cast<int64_t>(prm.table_width) << prm.page_shift;
-    if (!rows_fit_one_launch(prm.splits, prm.split_tokens, capacity, head_dim, elem)) return;
-    const int64_t span = lmin(static_cast<int64_t>(prm.splits) * prm.split_tokens, capacity);
+    const int64_t rows = static_cast<int64_t>(prm.batch) * kv_heads * prm.head_tiles;
+    if (!rows_fit_one_launch(rows, prm.reach, head_dim, elem, cus,
+                             may_share_prefixes(prm.host_prefix_runs, prm.host_bounds, prm.batch, slots)))
+        return;
+    const int64_t span = prm.reach;
+    max_waves = row_waves_for(rows, span * head_dim * elem * 2, imin(prm.head_tile, prm.group) * head_dim, max_waves, cus);
     int waves = static_cast<int>(lmin(max_waves, (span + kRowWaveTokens - 1) / kRowWaveTokens));
     while (waves > 1 && waves * (slot_bytes + stage_bytes) > 160 * 1024) --waves;
     prm.row_mode = 1;
@@ -1332,7 +1389,8 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
         prm.mid_grid = 0;
         prm.combine = prm.quarters_per_wg == 4;
     }
-    plan_rows(prm, head_dim, elem, combine_slot_bytes(head_dim), mfma_stage_bytes(head_dim, elem));
+    plan_rows(prm, kv_heads, head_dim, elem, combine_slot_bytes(head_dim), mfma_stage_bytes(head_dim, elem), cus,
+              prefix_slots(prm.group));
     plan_prefix_items(prm, prefix_slots(prm.group));
     plan_xcd(prm, kv_heads);
     // Where the merge reads its states from the XCD's L2 (plan_xcd), the fold
@@ -1353,12 +1411,12 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
 
 // Launch shape of the FP32 kernel (and whole rows, as for the matrix-core
 // kernel).
-inline void plan_fp32(PartialParams& prm, int kv_heads, int head_dim) {
+inline void plan_fp32(PartialParams& prm, int kv_heads, int head_dim, int cus = kMi355xCus) {
     const int gt = head_tile(prm.group, 8);
     prm.head_tile = gt;
     prm.head_tiles = (prm.group + gt - 1) / gt;
     choose_workgroup(prm, kv_heads, 8);
-    plan_rows(prm, head_dim, 4, row_slot_bytes_fp32(head_dim), 0, fp32_row_max_waves(gt));
+    plan_rows(prm, kv_heads, head_dim, 4, row_slot_bytes_fp32(head_dim), 0, cus, 1, fp32_row_max_waves(gt));
     plan_xcd(prm, kv_heads);
     const Grid grid = partial_grid(prm, kv_heads);
     prm.grid_x = grid.x;

@@ -262,8 +262,12 @@ class DecodePlan:
     def launches(self, q_dtype, kv_dtype=None):
         """Kernel launches ``run`` makes for q (and K/V) of these dtypes: 1 when the
         rows are small enough for one whole-row launch that writes the output
-        (the workspace is then left unwritten), else 2 (partition, merge)."""
+        (the workspace is then left unwritten), else 2 (partition, merge). Rows
+        that may form shared-prefix items keep two launches up to smaller
+        sizes, so with prefix runs the count comes from the launch plan."""
         layout = self.layout
+        if self._prefix_runs is not None:
+            return self.launch_plan(q_dtype, kv_dtype)["launches"]
         return self._extension.launch_count(q_dtype, q_dtype if kv_dtype is None else kv_dtype, layout.batch,
                                             layout.query_heads, layout.kv_heads, layout.head_dim, layout.page_size,
                                             self._table.shape[1], layout.physical_pages, self.splits,

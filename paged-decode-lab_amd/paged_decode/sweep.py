@@ -124,7 +124,7 @@ XCD = [
     _s("ragged B8 L4096", 8, 32, 8, 128, 16, "ragged:4096", 256),
 ]
 
-# Whole-row launches (plan_rows: rows of at most 128 KB of K and V), against
+# Whole-row launches (plan_rows: small rows, or rows enough for the CUs), against
 # the two-launch path through the stage entries (coarse factor 1).
 ROWS = [
     _s("fp32 B2 L256 Hq8/Hkv2 D64", 2, 8, 2, 64, 16, "uniform:256", 256, fmt="f32", coarse=(1,)),
@@ -134,6 +134,11 @@ ROWS = [
     _s("B64 L128 split 64", 64, 32, 8, 128, 16, "uniform:128", 64, coarse=(1,)),
     _s("mqa B128 L512 D64", 128, 16, 1, 64, 16, "uniform:512", 256, coarse=(1,)),
     _s("mqa B256 L256 D64", 256, 16, 1, 64, 16, "uniform:256", 256, coarse=(1,)),
+    _s("B32 L512", 32, 32, 8, 128, 16, "uniform:512", 256, coarse=(1,)),
+    _s("B32 L1024", 32, 32, 8, 128, 16, "uniform:1024", 256, coarse=(1,)),
+    _s("B256 L64", 256, 32, 8, 128, 16, "uniform:64", 256, coarse=(1,)),
+    _s("ragged B256 L256", 256, 32, 8, 128, 16, "ragged:256", 256, coarse=(1,)),
+    _s("ragged B256 L512", 256, 32, 8, 128, 16, "ragged:512", 256, coarse=(1,)),
 ]
 
 # Shared prefixes (plan_prefix_items): work lists whose partitions inside

@@ -170,3 +170,34 @@ def test_whole_rows_graph_replay(q_dtype):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(plan._out, eager)
+
+
+# (batch, query heads, KV heads, head_dim, tokens per row, launches on 256 CUs): rows on each side of the launch's
+# bounds (7/8 of the CUs for 256 KB, one per CU for 512 KB) and of its workgroup sizes (8 or 16 waves, 4, 2, 1).
+LARGE = [
+    (27, 32, 8, 128, 512, 2), (28, 32, 8, 128, 512, 1), (33, 32, 8, 128, 512, 1), (32, 32, 8, 128, 1024, 1),
+    (33, 32, 8, 128, 1024, 2), (32, 32, 8, 128, 1040, 2), (128, 16, 8, 64, 48, 1), (256, 8, 8, 64, 16, 1),
+    (256, 16, 8, 128, 33, 1), (255, 16, 1, 64, 512, 1), (257, 16, 1, 64, 1024, 1),
+]
+
+
+@pytest.mark.parametrize("shape", LARGE, ids=lambda s: "x".join(map(str, s[:5])))
+@pytest.mark.parametrize("q_dtype,kv_dtype", FORMATS[1:])
+def test_rows_that_fill_the_device(shape, q_dtype, kv_dtype):
+    batch, heads, kv_heads, dim, tokens, launches = shape
+    announce(f"whole rows, large batch q={q_dtype} kv={kv_dtype} shape={shape}")
+    width = (tokens + 15) // 16
+    pages = min(batch * width, 509)  # rows map the same pages in other orders, so the inputs stay small
+    layout = Layout(batch, heads, kv_heads, dim, 16, pages)
+    rng = np.random.default_rng(tokens)
+    table = np.stack([rng.permutation(pages)[:width] for _ in range(batch)]).astype(np.int32)
+    lengths = rng.integers(0, tokens + 1, size=batch, dtype=np.int32)
+    lengths[:2] = tokens, 0
+    table[:, 0] = np.arange(batch) % pages  # no common first page: no shared prefixes
+    (q, k, v), (k_scale, v_scale), exact = device_inputs(layout, q_dtype, kv_dtype, seed=batch)
+    plan = DecodePlan(layout, table, lengths, split_tokens=256)
+    plan._prefix_runs = None
+    if kv_dtype is None and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert plan.launches(q.dtype) == launches
+    out = plan.run(q, k, v, k_scale=k_scale, v_scale=v_scale).cpu().numpy()
+    assert_parity(out, dense_attention(*exact, table, lengths), torch.float16)
