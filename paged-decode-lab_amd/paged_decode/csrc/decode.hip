@@ -16,7 +16,7 @@
 //     in slot 4 * partition + quarter of the workspace. A workgroup gathers up
 //     to four KV heads (eight in the FP32 kernel) of the same tokens (their
 //     head slices of a token row are then read together) plus enough quarters
-//     to make eight waves, or fewer waves when eight-wave workgroups would
+//     to make four to eight waves, or fewer where such workgroups would
 //     leave most CUs idle. Waves
 //     do not synchronise while they stream; where a workgroup holds several
 //     quarters of one partition (few KV heads), one barrier at the end lets
@@ -26,7 +26,7 @@
 //     bounds reach, then a few tail workgroups for lengths that grew past
 //     them on the device.
 //       partial_mfma_kernel (q in FP16 or BF16; K/V in the same type or in
-//       OCP FP8): 16-token tiles; q.K^T and P.V on the matrix cores, online
+//       OCP FP8): pairs of 16-token tiles; q.K^T and P.V on the matrix cores, online
 //       softmax with one running max per head and lazy rescaling (the
 //       accumulators are rescaled only when a tile's max exceeds the running
 //       max by 2^8); each lane ends with its own slice of the state and
@@ -37,7 +37,7 @@
 //       combined with lane shuffles before the store.
 //     Page ids come from a 64-entry, lane-indexed window read once per wave
 //     and indexed with v_readlane; loads stream through a short register
-//     pipeline in fully unrolled blocks, K and V alike as whole token rows
+//     pipeline, K and V alike as whole token rows
 //     (K reaches the MFMA operand layout through LDS). Scores are kept in log2 units
 //     (scale * log2 e) and exponentiated with v_exp_f32.
 //  2. Merge: max-corrected combination of the live states of each (sequence,

@@ -313,20 +313,36 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
 // s, of tile token sigma(l % 16)), q in the B layout (lane l: query head
 // l % 16, zero past the group). K is loaded as whole token rows (16 bytes per
 // lane, full cache lines, like V) and reaches the A layout through a per-wave
-// LDS tile. With sigma(r) = r / 4 + 4 (r % 4) the result
-// leaves lane l with head n = l % 16 and tokens g, g + 4, g + 8, g + 12 of the
-// tile (g = l / 16): exactly the A operand of v_mfma_f32_16x16x16_{f16,bf16}
-// for P (row = head, k = 4 g + e <-> token g + 4 e), so the weights never
-// leave their lanes. V is loaded in the row layout -- load e covers tokens
-// 4 e .. 4 e + 3, lanes [16 r, 16 r + 16) token 4 e + r, VH consecutive dims
-// per lane -- so lane (g, n) holds tokens g + 4 e of dims n VH .. n VH + VH - 1,
-// and element j of its four V loads is the B operand of MFMA block j (column
-// n <-> dim n VH + j). P is split into high and low parts of the compute type
-// (two MFMAs per block), which keeps the weights exact to about 2^-22 (FP16)
-// or 2^-17 (BF16) relative. Each (head, dim) sum lives in exactly one lane:
-// lane (g, n) ends with heads 4 g .. 4 g + 3 of dims n VH .. n VH + VH - 1,
-// stored directly. One running max per head is shared by the wave, with lazy
-// rescaling as in the FP32 kernel.
+// LDS tile. With sigma(r) = r / 4 + 4 (r % 4) the result leaves lane l with
+// head n = l % 16 and tokens g, g + 4, g + 8, g + 12 of the tile (g = l / 16).
+// Tiles go in pairs: the scores of both are the A operand of
+// v_mfma_f32_16x16x32 for P (row = head, k = 8 g + 4 h + e <-> token g + 4 e of
+// tile h), so the weights never leave their lanes. V is loaded in the row
+// layout -- load e covers tokens 4 e .. 4 e + 3, lanes [16 r, 16 r + 16) token
+// 4 e + r, VH consecutive dims per lane -- so lane (g, n) holds tokens g + 4 e
+// of dims n VH .. n VH + VH - 1, and element j of a pair's eight V loads is the
+// B operand of MFMA block j (column n <-> dim n VH + j). P is split into high
+// and low parts of the compute type (two MFMAs per block), which keeps the
+// weights exact to about 2^-22 (FP16) or 2^-17 (BF16) relative. Each (head,
+// dim) sum lives in exactly one lane: lane (g, n) ends with heads 4 g ..
+// 4 g + 3 of dims n VH .. n VH + VH - 1, stored directly. One running max per
+// head is shared by the wave, with lazy rescaling as in the FP32 kernel.
+//
+// What bounds it is the time a wave does not have loads in flight. With the
+// waves of a grid all started together, blocks of loads followed by their
+// computation left the memory idle while every wave computed: FP8 B16 L4096
+// (ragged, 90 MB) ran 26 us where a plain gather of as many pages takes 15. So
+// a pair's K is requested again (the next pair's) as soon as it is scored and
+// its V as soon as it is summed; the descriptors' range check (tile_buffer)
+// replaces clamped addresses, the softmax runs once per pair, and P.V takes
+// 32 tokens per MFMA: about 115 vector instructions per 32 FP16 tokens, 370
+// before. Measured on MI355X, decode call, us (graph, K/V rotated past the
+// Infinity Cache; blocks of two or four tiles, FP8 -> pairs): FP8 B16 L4096
+// ragged 33.1 -> 25.3, B32 51.4 -> 39.5, B64 L8192 164.6 -> 143.2, B4 L4096 15.6 ->
+// 14.0; FP16 B1 L4096 10.2 -> 9.3, B4 18.1 -> 17.7, B8 ragged 22.9 -> 21.3, B16
+// ragged 39.5 -> 36.7; FP16 MQA B256 L2048 31.6 -> 28.2; B64 L8192 ragged 231 ->
+// 227. Two pairs in flight per wave (173 VGPRs and more, two waves per SIMD)
+// were slower: FP8 B4 15.3, FP16 B4 18.7, B16 ragged FP8 27.8 against 26.9.
 //
 // FP8 K/V (OCP e4m3 or e5m2) are loaded as bytes and converted to the compute
 // type after they arrive; both formats convert exactly. The per-tensor scales
@@ -336,23 +352,29 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
 enum KvFormat { kKvNative = 0, kKvE4M3 = 1, kKvE5M2 = 2 };
 
 
-// N stored words from src. kStream marks 16-byte loads non-temporal (see
-// plan_mfma for when that is used).
+// Buffer descriptor of `bytes` bytes at base (uniform over the wave): loads
+// from byte offset `bytes` on return zeros and touch no memory.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const char* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00027000);
+}
+
+// N stored words at byte offset `offset` of a buffer. kStream marks 16-byte
+// loads non-temporal (see plan_mfma for when that is used).
 template <int N, bool kStream>
-__device__ __forceinline__ void load_words(const char* src, uint32_t (&w)[N]) {
+__device__ __forceinline__ void load_words(__amdgpu_buffer_rsrc_t buffer, uint32_t offset, uint32_t (&w)[N]) {
+    constexpr int kAux = kStream && N == 4 ? 2 : 0;
     if constexpr (N == 4) {
-        const u32x4 x = kStream ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src))
-                                : *reinterpret_cast<const u32x4*>(src);
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(buffer, offset, 0, kAux);
         w[0] = x[0];
         w[1] = x[1];
         w[2] = x[2];
         w[3] = x[3];
     } else if constexpr (N == 2) {
-        const u32x2 x = *reinterpret_cast<const u32x2*>(src);
+        const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(buffer, offset, 0, kAux);
         w[0] = x[0];
         w[1] = x[1];
     } else {
-        w[0] = *reinterpret_cast<const uint32_t*>(src);
+        w[0] = __builtin_amdgcn_raw_buffer_load_b32(buffer, offset, 0, kAux);
     }
 }
 
@@ -370,11 +392,12 @@ struct Compute<_Float16> {
         return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c, 0,
                                                      0, 0);
     }
-    // Nearest 16-bit value of x, and that value back as FP32.
-    static __device__ __forceinline__ uint16_t round(float x, float& back) {
-        const _Float16 h = static_cast<_Float16>(x);
-        back = static_cast<float>(h);
-        return __builtin_bit_cast(uint16_t, h);
+    // Nearest 16-bit values of (a, b), packed, and those values back as FP32.
+    static __device__ __forceinline__ uint32_t round(float a, float b, float& back_a, float& back_b) {
+        const f16x2 h = __builtin_convertvector((f32x2{a, b}), f16x2);
+        back_a = static_cast<float>(h[0]);
+        back_b = static_cast<float>(h[1]);
+        return __builtin_bit_cast(uint32_t, h);
     }
     // Bytes 2 HIGH, 2 HIGH + 1 of an FP8 word as a packed pair (exact).
     template <int KVF, bool HIGH>
@@ -396,10 +419,12 @@ struct Compute<__bf16> {
         return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c,
                                                          0, 0, 0);
     }
-    static __device__ __forceinline__ uint16_t round(float x, float& back) {
-        const __bf16 h = static_cast<__bf16>(x);
-        back = static_cast<float>(h);
-        return __builtin_bit_cast(uint16_t, h);
+    static __device__ __forceinline__ uint32_t round(float a, float b, float& back_a, float& back_b) {
+        const bf16x2 h = __builtin_convertvector((f32x2{a, b}), bf16x2);
+        const uint32_t bits = __builtin_bit_cast(uint32_t, h);
+        back_a = __builtin_bit_cast(float, bits << 16);
+        back_b = __builtin_bit_cast(float, bits & 0xFFFF0000u);
+        return bits;
     }
     template <int KVF, bool HIGH>
     static __device__ __forceinline__ uint32_t from_fp8(uint32_t word) {
@@ -430,9 +455,10 @@ __device__ __forceinline__ void to_compute(const uint32_t (&raw)[N], uint32_t (&
 // packed words), packed as an MFMA operand (k = load index).
 template <int VH>
 __device__ __forceinline__ u32x2 v_operand(const uint32_t (&v)[4][VH / 2], int j) {
-    const uint32_t d0 = v[0][j / 2], d1 = v[1][j / 2], d2 = v[2][j / 2], d3 = v[3][j / 2];
-    if (j % 2 == 0) return u32x2{(d0 & 0xFFFFu) | (d1 << 16), (d2 & 0xFFFFu) | (d3 << 16)};
-    return u32x2{(d0 >> 16) | (d1 & 0xFFFF0000u), (d2 >> 16) | (d3 & 0xFFFF0000u)};
+    constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;  // halves of (second, first)
+    const uint32_t sel = j % 2 == 0 ? kLow : kHigh;
+    return u32x2{__builtin_amdgcn_perm(v[1][j / 2], v[0][j / 2], sel),
+                 __builtin_amdgcn_perm(v[3][j / 2], v[2][j / 2], sel)};
 }
 
 // LDS slot of the quarter combine: one quarter's state of one (KV head,
@@ -450,8 +476,8 @@ struct CombineSlot {
 // kFold: what the workgroup stores -- 0 one state per wave; 1 one state per
 // qw quarters of a partition (quarter combine); 2 the output rows of a whole
 // row's states (whole-row launch, up to kRowMaxWaves waves: 1024 lanes).
-template <typename QT, int KVF, int D, int GT, int PD, int NC, int kStream, int kFold, int kList>
-__global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
+template <typename QT, int KVF, int D, int GT, int NB, int kStream, int kFold, int kList>
+__global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave * 8, KVF == kKvNative ? 3 : 4)
     partial_mfma_kernel(const PartialParams p) {
     using C = Compute<QT>;
     constexpr int ES = KVF == kKvNative ? 2 : 1;  // stored bytes per K/V element
@@ -460,6 +486,8 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
     constexpr int VI = 4;                         // V loads per tile
     constexpr int VW = VH * ES / 4;               // stored words per V load
     static_assert(GT <= 16, "one MFMA column block holds at most 16 query heads");
+    constexpr int kPair = 2;
+    constexpr int kPairTokens = kPair * kTileTokens;
 
     // K is loaded whole rows at a time (KR lanes x 16 bytes per token, TK
     // tokens per load, KL loads per tile) and turned into the q.K^T operand
@@ -479,10 +507,15 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
     char* const k_stage = lds;
     char* const combine_lds = lds + mfma_stage_bytes(D, ES) * (blockDim.x / kWave);
 
-    struct Tile {
-        uint32_t k[KL][4];
-        uint32_t v[VI][VW];
-        uint32_t live;
+    // Tiles are read and scored kPair at a time: one softmax step, and P.V
+    // over all their tokens in one 16x16x32 MFMA per block.
+    struct Request {  // where a pair of tiles lies
+        uint64_t base[kPair];
+        uint32_t bytes[kPair];  // of each tile's live rows (0: nothing to read)
+    };
+    struct Pair {
+        uint32_t k[kPair][KL][4];
+        uint32_t v[kPair][VI][VW];
     };
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -593,8 +626,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
 
     const char* k_head = static_cast<const char*>(p.k) + static_cast<size_t>(w.kv_head) * D * ES;
     const char* v_head = static_cast<const char*>(p.v) + static_cast<size_t>(w.kv_head) * D * ES;
-    const char* park = q_row;  // dead tiles read the wave's own q row: mapped, D * 2 bytes
-    const uint32_t v_lane_bytes = static_cast<uint32_t>(n) * VH * ES;
+    // This lane's bytes of row 0 of a tile's first K load and first V load.
+    const uint32_t k_lane = tile_row_offset(p, lane / KR, static_cast<uint32_t>(lane % KR) * 16u);
+    const uint32_t v_lane = tile_row_offset(p, g, static_cast<uint32_t>(n) * VH * ES);
     const int k_row_token = k_token_of_row(n);
     int rb = w.wb, re = w.wb;
     // The pass: its page-table row, its token end, and whether this lane's
@@ -603,36 +637,53 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
     int pass_end = w.we;
     bool col_on = !grouped || ((own >> col_member) & 1u) == 0;
 
-    auto issue = [&](Tile& tl, int t0, int ids, int win) {
-        const TileSpan span = tile_span(p, t0, kTileTokens, rb, re, win);
-        const int page = __builtin_amdgcn_readlane(ids, span.slot);
-        const bool ok = tile_live(p, t0, re, page);
-        tl.live = ok;
-        const uint64_t page_off = tile_page_offset(p, ok, page);
-        const char* kp = ok ? k_head + page_off : park;
-        const char* vp = ok ? v_head + page_off : park;
-        const uint32_t k_lane_bytes = static_cast<uint32_t>(lane % KR) * 16u;
+    auto locate = [&](int t0) {
+        Request rq;
 #pragma unroll
-        for (int s = 0; s < KL; ++s)
-            load_words<4, kStreamK>(kp + token_offset(p, ok, t0 + TK * s + lane / KR, span, k_lane_bytes), tl.k[s]);
+        for (int h = 0; h < kPair; ++h) {
+            const int t = t0 + h * kTileTokens;
+            const int page = __builtin_amdgcn_readlane(window_ids, tile_slot(p, t, window));
+            rq.base[h] = tile_base(p, page, t);
+            rq.bytes[h] = tile_bytes(p, tile_live(p, t, re, page), t, re);
+        }
+        return rq;
+    };
+    auto load_k = [&](Pair& pr2, const Request& rq) {
 #pragma unroll
-        for (int e = 0; e < VI; ++e)
-            load_words<VW, (kStream >= 1)>(vp + token_offset(p, ok, t0 + 4 * e + g, span, v_lane_bytes), tl.v[e]);
+        for (int h = 0; h < kPair; ++h) {
+            const __amdgpu_buffer_rsrc_t kb = tile_buffer(k_head + rq.base[h], rq.bytes[h]);
+#pragma unroll
+            for (int s = 0; s < KL; ++s)
+                load_words<4, kStreamK>(kb, k_lane + tile_row_offset(p, TK * s, 0), pr2.k[h][s]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_v = [&](Pair& pr2, const Request& rq) {
+#pragma unroll
+        for (int h = 0; h < kPair; ++h) {
+            const __amdgpu_buffer_rsrc_t vb = tile_buffer(v_head + rq.base[h], rq.bytes[h]);
+#pragma unroll
+            for (int e = 0; e < VI; ++e)
+                load_words<VW, (kStream >= 1)>(vb, v_lane + tile_row_offset(p, 4 * e, 0), pr2.v[h][e]);
+        }
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    auto consume = [&](const Tile& tl, int t0) {
+    // Raw scores of tile h of the pair at t0: K through the wave's LDS tile
+    // into the operand layout, then q.K^T.
+    auto score = [&](const Pair& pr2, int h) {
         f32x4 sc = {0.0f, 0.0f, 0.0f, 0.0f};
         char* stage = k_stage + wave * (kTileTokens * kStageRow);
         __builtin_amdgcn_wave_barrier();  // the previous tile's reads are issued before these writes
 #pragma unroll
         for (int s = 0; s < KL; ++s) {
+            const uint32_t* kw = pr2.k[h][s];
             char* dst = stage + (TK * s + lane / KR) * kStageRow + (lane % KR) * 16;
             if constexpr (kStageRow % 16 == 0) {
-                *reinterpret_cast<u32x4*>(dst) = u32x4{tl.k[s][0], tl.k[s][1], tl.k[s][2], tl.k[s][3]};
+                *reinterpret_cast<u32x4*>(dst) = u32x4{kw[0], kw[1], kw[2], kw[3]};
             } else {  // FP8 rows are 8-byte aligned
-                reinterpret_cast<u32x2*>(dst)[0] = u32x2{tl.k[s][0], tl.k[s][1]};
-                reinterpret_cast<u32x2*>(dst)[1] = u32x2{tl.k[s][2], tl.k[s][3]};
+                reinterpret_cast<u32x2*>(dst)[0] = u32x2{kw[0], kw[1]};
+                reinterpret_cast<u32x2*>(dst)[1] = u32x2{kw[2], kw[3]};
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -649,18 +700,32 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
                 sc = C::qk(u32x4{kq[0], kq[1], kq[2], kq[3]}, qb[s], sc);
             }
         }
-        float x[4];
+        return sc;
+    };
+
+    // Softmax and P.V of the pair at t0, whose scores are sc.
+    auto accumulate = [&](Pair& pr2, const Request& rq, f32x4 (&sc)[kPair], int t0) {
         float mx = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int t = t0 + g + 4 * e;
-            const bool valid = (tl.live != 0u) & (t >= rb) & (t < re) & (t < col_end) & col_on;
-            x[e] = valid ? sc[e] : -INFINITY;
-            mx = fmaxf(mx, x[e]);
+        for (int h = 0; h < kPair; ++h) {
+            const int t1 = t0 + h * kTileTokens;
+            // Whole tiles of an ungrouped item need no mask.
+            if (grouped || rq.bytes[h] == 0u || t1 < rb || t1 + kTileTokens > re) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = t1 + g + 4 * e;
+                    const bool valid = (rq.bytes[h] != 0u) & (t >= rb) & (t < re) & (t < col_end) & col_on;
+                    sc[h][e] = valid ? sc[h][e] : -INFINITY;
+                    // Rows before the range are another quarter's: their V stays out of this one's sums.
+#pragma unroll
+                    for (int i = 0; i < VW; ++i) pr2.v[h][e][i] = t >= rb ? pr2.v[h][e][i] : 0u;
+                }
+            }
+            mx = fmaxf(mx, fmaxf(fmaxf(sc[h][0], sc[h][1]), fmaxf(sc[h][2], sc[h][3])));
         }
-        const float tile_max = max_over_lane_groups(mx) * p.scale_log2;
-        if (__any((n < GT * pr.members) & (tile_max > m_head + kRescaleSlack))) {
-            const float m_new = fmaxf(m_head, tile_max);
+        const float pair_max = max_over_lane_groups(mx) * p.scale_log2;
+        if (__builtin_amdgcn_ballot_w64((n < GT * pr.members) & (pair_max > m_head + kRescaleSlack)) != 0) {
+            const float m_new = fmaxf(m_head, pair_max);
             const float alpha = fast_exp2(m_head - m_new);
             m_head = m_new;
             l_part *= alpha;
@@ -672,31 +737,44 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
                 for (int j = 0; j < VH; ++j) acc[j][i] *= a;
             }
         }
-        uint16_t hi_bits[4], lo_bits[4];
+        // P in high and low parts, k = 8 g + 4 h + e <-> token g + 4 e of tile h.
+        u32x4 p_hi, p_lo;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float wt = fast_exp2(fmaf(x[e], p.scale_log2, -m_head));
-            l_part += wt;
-            float back, unused;
-            hi_bits[e] = C::round(wt, back);
-            lo_bits[e] = C::round(wt - back, unused);
+        for (int h = 0; h < kPair; ++h) {
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) {
+                const float w0 = fast_exp2(fmaf(sc[h][e], p.scale_log2, -m_head));
+                const float w1 = fast_exp2(fmaf(sc[h][e + 1], p.scale_log2, -m_head));
+                l_part += w0;
+                l_part += w1;
+                float back0, back1, unused0, unused1;
+                p_hi[2 * h + e / 2] = C::round(w0, w1, back0, back1);
+                p_lo[2 * h + e / 2] = C::round(w0 - back0, w1 - back1, unused0, unused1);
+            }
         }
-        const u32x2 p_hi = {hi_bits[0] | (static_cast<uint32_t>(hi_bits[1]) << 16),
-                            hi_bits[2] | (static_cast<uint32_t>(hi_bits[3]) << 16)};
-        const u32x2 p_lo = {lo_bits[0] | (static_cast<uint32_t>(lo_bits[1]) << 16),
-                            lo_bits[2] | (static_cast<uint32_t>(lo_bits[3]) << 16)};
-        uint32_t vq[VI][VH / 2];
+        // One stored word of every V load at a time, so that only its converted
+        // form is live (FP8: the words of 4 of the lane's dims become 8 of them).
+        constexpr int kWordDims = 4 / ES;
 #pragma unroll
-        for (int e = 0; e < VI; ++e) {
-            uint32_t raw[VW];
+        for (int w4 = 0; w4 < VW; ++w4) {
+            uint32_t vq[kPair][VI][kWordDims / 2];
 #pragma unroll
-            for (int i = 0; i < VW; ++i) raw[i] = (KVF == kKvNative || tl.live) ? tl.v[e][i] : 0u;  // FP8 park bytes may decode to NaN
-            to_compute<QT, KVF, VW>(raw, vq[e]);
+            for (int h = 0; h < kPair; ++h)
+#pragma unroll
+                for (int e = 0; e < VI; ++e) {
+                    const uint32_t raw[1] = {pr2.v[h][e][w4]};
+                    to_compute<QT, KVF, 1>(raw, vq[h][e]);
+                }
+#pragma unroll
+            for (int j = 0; j < kWordDims; ++j) {
+                const u32x2 v0 = v_operand<kWordDims>(vq[0], j), v1 = v_operand<kWordDims>(vq[1], j);
+                const u32x4 vo = {v0[0], v0[1], v1[0], v1[1]};
+                f32x4& sum = acc[w4 * kWordDims + j];
+                sum = C::qk(p_hi, vo, sum);
+                sum = C::qk(p_lo, vo, sum);
+            }
+            if constexpr (KVF != kKvNative) __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int j = 0; j < VH; ++j) acc[j] = C::pv(p_hi, v_operand<VH>(vq, j), acc[j]);
-#pragma unroll
-        for (int j = 0; j < VH; ++j) acc[j] = C::pv(p_lo, v_operand<VH>(vq, j), acc[j]);
     };
 
     uint32_t pending = own;
@@ -707,15 +785,31 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * kRowMaxWaves : kWave * 8)
                 window_ids = pass_pages[window_entry(p, window, lane)];
             }
             re = min(pass_end, (window + kWave) << p.page_shift);
-            for (int s0 = rb & ~(kTileTokens - 1); s0 < re; s0 += NC * kTileTokens) {
-                Tile buf[PD + 1];
+            // A ring of NB pairs. Once a pair's K is scored, the K of the pair
+            // NB on is requested into its registers, and likewise V, so that
+            // loads are in flight while the wave computes. (Requests past the
+            // range are empty rather than skipped, and the loop has one exit:
+            // the compiler then counts the loads outstanding at every wait.)
+            Pair ring[NB];
+            Request at[NB];
+            int s0 = rb & ~(kTileTokens - 1);
 #pragma unroll
-                for (int n0 = 0; n0 < PD; ++n0) issue(buf[n0], s0 + n0 * kTileTokens, window_ids, window);
+            for (int c = 0; c < NB; ++c) {
+                at[c] = locate(s0 + c * kPairTokens);
+                load_k(ring[c], at[c]);
+                load_v(ring[c], at[c]);
+            }
+            for (; s0 < re; s0 += NB * kPairTokens) {
 #pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    if (s0 + c * kTileTokens >= re) break;
-                    if (c + PD < NC) issue(buf[(c + PD) % (PD + 1)], s0 + (c + PD) * kTileTokens, window_ids, window);
-                    consume(buf[c % (PD + 1)], s0 + c * kTileTokens);
+                for (int c = 0; c < NB; ++c) {
+                    f32x4 sc[kPair];
+#pragma unroll
+                    for (int h = 0; h < kPair; ++h) sc[h] = score(ring[c], h);
+                    const Request next = locate(s0 + (NB + c) * kPairTokens);
+                    load_k(ring[c], next);
+                    accumulate(ring[c], at[c], sc, s0 + c * kPairTokens);
+                    load_v(ring[c], next);
+                    at[c] = next;
                 }
             }
         }
@@ -851,22 +945,8 @@ constexpr int kFp32BlockChunks = 16;
 // Whole-row FP32 launches give each wave a slice of a few chunks (16 tokens
 // at most rows' sizes): a block of four keeps the straight-line code short.
 constexpr int kFp32RowBlockChunks = 4;
-// Matrix-core kernel: 16-token tiles issued ahead of the one being consumed,
-// and tiles per straight-line block (with 2 and 2, each block's two tiles are
-// requested together and consumed in order). Short blocks keep the kernel's
-// code small: with 8 waves per CU running through cold straight-line code,
-// instruction fetch is on the critical path (two-tile blocks measured 1 us
-// faster per Llama-3-8B-shape call than eight-tile blocks, same loads).
-constexpr int kMfmaPrefetch = 2;
-constexpr int kMfmaBlock = 2;
-// FP8 K/V tiles are half the bytes: a 64-token quarter's four tiles are all
-// requested at once, in one block. Measured on MI355X (decode call, us), 2 and
-// 2 -> 4 and 4: B1 L4096 10.7 -> 10.2, B16 L4096 32.5 -> 32.1, MQA B128 L1024
-// D64 12.03 -> 11.90, Llama-3-8B B4 L4096 14.7 -> 14.7. Whole-row launches
-// keep 2 and 2: at 1024 lanes their kernel has 128 VGPRs, and four tiles in
-// flight spilled.
-constexpr int kMfmaPrefetchFp8 = 4;
-constexpr int kMfmaBlockFp8 = 4;
+// Matrix-core kernel: pairs of 16-token tiles in flight per wave.
+constexpr int kMfmaRing = 1;
 
 // Compute units of the current device, read once per device.
 inline int device_compute_units() {
@@ -893,22 +973,20 @@ int launch_mfma(const PartialParams& prm, int kv_heads, hipStream_t stream) {
     const dim3 block(partial_threads(prm));
     const size_t lds = static_cast<size_t>(mfma_lds_bytes(prm, D, KVF == kKvNative ? 2 : 1));
     const int kind = grid_kind(prm);
-    constexpr int kPD = KVF == kKvNative ? kMfmaPrefetch : kMfmaPrefetchFp8;
-    constexpr int kNC = KVF == kKvNative ? kMfmaBlock : kMfmaBlockFp8;
     // Whole-row launches are rectangular (one workgroup per row).
 #define PD_LAUNCH_MFMA(MODE, FOLD)                                                                                \
     do {                                                                                                          \
         if constexpr (FOLD == 2)                                                                                  \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaPrefetch, kMfmaBlock, MODE, 2, kGridRect>), \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, 2, kGridRect>), \
                                grid, block, lds, stream, prm);                                                    \
         else if (kind == kGridList)                                                                               \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kPD, kNC, MODE, FOLD, kGridList>), grid,      \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, FOLD, kGridList>), grid,      \
                                block, lds, stream, prm);                                                          \
         else if (kind == kGridRectTails)                                                                          \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kPD, kNC, MODE, FOLD, kGridRectTails>), grid, \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, FOLD, kGridRectTails>), grid, \
                                block, lds, stream, prm);                                                          \
         else                                                                                                      \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kPD, kNC, MODE, FOLD, kGridRect>), grid,      \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, FOLD, kGridRect>), grid,      \
                                block, lds, stream, prm);                                                          \
     } while (0)
 #define PD_LAUNCH_MFMA_FOLDS(MODE)                      \

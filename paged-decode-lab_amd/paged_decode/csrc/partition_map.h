@@ -470,6 +470,27 @@ PD_HD uint32_t token_offset(const PartialParams& p, bool ok, int t, const TileSp
     return ok ? static_cast<uint32_t>(tk & ((1 << p.page_shift) - 1)) * p.token_bytes + lane_bytes : lane_bytes;
 }
 
+// The matrix-core kernel reads a tile through a buffer descriptor: base
+// tile_base bytes from the head's first page (the tile's first token, which a
+// tile never leaves the page of), tile_bytes long, row i of the tile at
+// tile_row_offset(i). Rows from the range's end re on, and every row of a tile
+// that is not live (tile_live), lie past the descriptor's end: the hardware's
+// range check returns zeros for them and reads nothing, so a row needs no
+// clamped address of its own.
+PD_HD int tile_slot(const PartialParams& p, int t0, int window) {
+    return imin((t0 >> p.page_shift) - window, kWave - 1);
+}
+PD_HD uint64_t tile_base(const PartialParams& p, int page, int t0) {
+    return static_cast<uint64_t>(static_cast<uint32_t>(page)) * static_cast<uint32_t>(p.page_bytes) +
+           static_cast<uint32_t>(t0 & ((1 << p.page_shift) - 1)) * p.token_bytes;
+}
+PD_HD uint32_t tile_bytes(const PartialParams& p, bool ok, int t0, int re) {
+    return ok ? static_cast<uint32_t>(imin(kTileTokens, re - t0)) * p.token_bytes : 0u;
+}
+PD_HD uint32_t tile_row_offset(const PartialParams& p, int row, uint32_t lane_bytes) {
+    return static_cast<uint32_t>(row) * p.token_bytes + lane_bytes;
+}
+
 // Tile token whose K the q.K^T A operand of matrix-core lane row r (r = lane
 // % 16) holds: sigma(r) = r / 4 + 4 (r % 4), which leaves the scores of
 // tokens g, g + 4, g + 8, g + 12 in lane group g, the P.V A layout.
@@ -692,8 +713,8 @@ inline int partial_threads(const PartialParams& prm) {
     return kWave * prm.heads_per_wg * prm.tiles_per_wg * prm.quarters_per_wg;
 }
 
-// KV heads per workgroup of the matrix-core kernel, at most (FP32 kernel: 8).
-constexpr int kMfmaWorkgroupHeads = 4;
+// KV heads per workgroup of a small grid of the matrix-core kernel, at most.
+constexpr int kMfmaSmallGridHeads = 4;
 
 // LDS bytes of one wave's K tile in the matrix-core kernel: 16 token rows of
 // head_dim elements of elem bytes, each padded by one operand read (16 bytes
@@ -708,6 +729,7 @@ constexpr int combine_slot_bytes(int head_dim) { return 2 * 16 * 4 + (head_dim /
 // Waves of a whole-row workgroup, at most: the kernel is built for 1024-lane
 // workgroups in that mode.
 constexpr int kRowMaxWaves = 16;
+constexpr int row_max_waves(int head_dim) { return head_dim > 64 ? 12 : kRowMaxWaves; }  // matrix-core kernel
 
 // Dynamic LDS of a matrix-core launch: every wave's K tile, then the combine
 // slots ([waves / qw][qw - 1]) when the launch combines quarters, or one slot
@@ -922,32 +944,23 @@ inline int prefix_finer_split(int c, const int32_t* runs, const int32_t* bounds,
 // rounding. Longer partitions mean longer waves, so the per-wave latencies
 // (page ids and first K/V loads, the last tile, the state stores) and the
 // merge's states weigh less per byte -- while the grid keeps enough waves to
-// cover the device. c doubles while a wave would read at most
-// kCoarseWaveBytes of K and V and the live partitions, as far as the host
-// bounds tell, still give kCoarseWavesPerCu waves per CU. A call without
-// bounds keeps its split: counting every allocated partition as live
-// over-coarsens plans that reserve context (Llama-3-8B B4 L4096 with 4x
-// reserved: 21.7 -> 28.4 us). Measured on MI355X (decode call, us, graph of 200 calls, K/V
-// rotated over 2 GiB; the split the rule picks in brackets):
-//   ragged + shared-prefix B16, page 32, split 128: 40.8 -> 31.9 [512]
-//     (1024: 32.5, 2048: 37.7);
-//   uniform B16 / B32 L4096, 8 KV heads, split 256: 53.6 -> 48.0 [1024] /
-//     102.6 -> 90.6 [1024]; B64 L2048: 101.6 -> 91.3 [1024];
-//   FP8 K/V B16 L4096: 36.6 -> 32.4 [1024]; MQA B512 L1024 D64: 36.8 ->
-//     32.7 [1024];
-//   the reference's B16 L4096 batch: 44.3 -> 41.1 [512] (1024: 39.3);
-//   32K-context MHA at split 128: 93.3 -> 85.7 [1024];
-//   grids of at most eight waves per CU keep their split: doubling it made
-//     the Llama-3-8B B4 L4096 FP8 call 14.8 -> 17.9, MQA B128 L1024 14.1 ->
-//     16.3, the reference's B4 batch 14.7 -> 16.2 (FP16 Llama-3-8B: 17.4 ->
-//     17.3).
-// Going on to four waves per CU helped some shapes and hurt others badly
-// (FP16 B2 L8192 17.6 -> 17.2; FP8 K/V B16 L4096 32.5 -> 47.2, MQA B256
-// L1024 20.2 -> 25.0, FP16 B6 L4096 22.6 -> 23.0), so the rule stops at eight.
+// cover the device. c doubles while a wave would read at most kCoarseWaveBytes
+// of K and V and the live partitions, as far as the host bounds tell, still
+// give enough waves per CU. A call without bounds keeps its split: counting
+// every allocated partition as live over-coarsens plans that reserve context
+// (Llama-3-8B B4 L4096 with 4x reserved: 21.7 -> 28.4 us). Measured on MI355X
+// (decode call, us, graph, K/V rotated past the Infinity Cache; split 256 unless
+// named; the split the rule picks in brackets): uniform B16 L4096 53.6 -> 48.0
+// [1024], the ragged + shared B16 batch at split 128 40.8 -> 31.9 [512]; with
+// at least 6 instead of 8 waves per CU ragged B16 L4096 40.5 -> 36.7, FP8 K/V
+// 30.5 -> 27.6, GQA 5 40.7 -> 36.9, FP8 B32 L4096 45.6 -> 43.7, D 64 43.0 -> 40.8,
+// but equal lengths B6 L4096 22.8 -> 23.8 and, at 5, the work list of a ragged +
+// shared B16 batch 46.3 -> 57.1, so equal lengths and work lists keep 8.
 // Whole-row calls and FP32 inputs keep the caller's split. With prefix runs
 // (`slots` members per shared-prefix item, pages of 1 << page_shift tokens)
 // prefix_finer_split may halve c.
 constexpr int64_t kCoarseWaveBytes = 128 * 1024;
+constexpr int kCoarseWavesRagged = 6;
 
 struct KernelSplit {
     int splits, split_tokens;
@@ -960,18 +973,25 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
     const int64_t capacity = static_cast<int64_t>(table_width) * page_size;
     // Tokens the caller's partitions reach; no partition of a coarser split goes past them.
     const int64_t reach = lmin(static_cast<int64_t>(splits) * split_tokens, capacity);
-    // Whether partitions of `span` tokens leave enough waves per CU. Shared-
-    // prefix items are not counted: measured with them, the ragged + shared
-    // B16 workload ran 27.2 us per staged call at the 512-token partitions
-    // this count picks and 32.5 us at 256 tokens, where counting the items'
-    // waves against 8 per CU would have stopped.
+    // Whether partitions of `span` tokens leave enough waves per CU:
+    // kCoarseWavesPerCu, or kCoarseWavesRagged for lengths that are neither
+    // equal nor ragged enough for a work list. Shared-prefix items are not
+    // counted: measured with them, the ragged + shared B16 workload ran 27.2 us
+    // per staged call at the 512-token partitions this count picks and 32.5 us
+    // at 256 tokens, where counting the items' waves against 8 per CU would
+    // have stopped.
     auto enough = [&](int64_t span) {
-        int64_t parts = 0;
+        int64_t parts = 0, most = 0, fewest = splits;
         for (int b = 0; b < batch; ++b) {
             const int64_t bound = lmin(reach, length_bounds[b] < 0 ? 0 : length_bounds[b]);
-            parts += (bound + span - 1) / span;
+            const int64_t live = (bound + span - 1) / span;
+            parts += live;
+            most = live > most ? live : most;
+            fewest = lmin(fewest, live);
         }
-        return parts * kQuarters * kv_heads * head_tiles >= static_cast<int64_t>(kCoarseWavesPerCu) * cus;
+        const bool ragged = fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
+        return parts * kQuarters * kv_heads * head_tiles >=
+               static_cast<int64_t>(ragged ? kCoarseWavesRagged : kCoarseWavesPerCu) * cus;
     };
     int c = 1;
     while (2 * c <= splits) {
@@ -1255,62 +1275,50 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     prm.head_tile = gt;
     prm.head_tiles = (prm.group + gt - 1) / gt;
     prefer_work_list_for_prefixes(prm, kv_heads, prefix_slots(prm.group), cus);
-    choose_workgroup(prm, kv_heads, kMfmaWorkgroupHeads);
-    // A grid of at most half as many 8-wave workgroups as CUs leaves most CUs
-    // idle, and each busy CU can keep only so many loads in flight. The same
-    // waves then go in smaller workgroups, the largest of 4, 2 or 1 waves
-    // that still gives two workgroups per CU (else 1 wave). Measured on
-    // MI355X, Llama-3-8B geometry (decode call, us):
-    //   B1 L4096 (64 workgroups of 8 waves): 12.4 -> 10.2 with 1 wave;
-    //   B1 L2048: 11.7 -> 9.9; FP8 B1 L4096: 12.6 -> 10.6-11.1;
-    //   B2 L4096 and B1 L8192 (128 workgroups): 13.2 -> 12.9 and
-    //   13.65 -> 13.1 with 2 waves.
-    // At 192 workgroups (B3 L4096) every smaller shape was slower (14.95 ->
-    // 15.3-19.0), so larger grids keep 8 waves.
+    // Workgroups of 2 KV heads x 2 quarters (4 waves) where a head's slice of a
+    // token row is 256 bytes or more (or there are no more heads), else of 4 KV
+    // heads x 2 quarters (8 waves), where the heads allow it (6 waves for heads of several tiles, three of
+    // which then still take two quarters); a KV head count with no such divisor
+    // keeps its whole token row in one workgroup of one quarter when it fits.
+    // The 16-bit
+    // D 128 kernels need up to 168 VGPRs (three waves per SIMD; their loads
+    // overlap their own computation), so three 4-wave workgroups share a CU,
+    // where an 8-wave workgroup would hold one alone; the others fit 128, and
+    // read half as many bytes of a row per head. Measured on MI355X (decode
+    // call, us, graph; 4 KV heads x 2 quarters in 8 waves / x 1 in 4 / 2 x 2 in
+    // 4): B64 L6144 276.5 / 276.3 / 269.4, B64 L8192 ragged 226.6 / 248.8 /
+    // 226.9, B16 L8192 92.7 / 96.2 / 92.8, page lists loaded on the device (no
+    // bounds) B32 L4096 87.8 / 79.8 / 77.6; FP8 K/V (8 waves / 2 x 2 in 4) B64
+    // L8192 ragged 143.2 / 155.8, B32 L4096 ragged 39.5 / 43.4, B32 L8192 99.3 /
+    // 102.1. B16 ragged with 5 KV heads 28.6 whole, 30.4 as 1 x 4; B8 with 7 KV
+    // heads 25.1 and 26.1.
+    const bool wide = head_dim * elem >= 256;
+    choose_workgroup(prm, kv_heads, wide ? 2 : 4, !wide && kv_heads > 2 ? 8 : prm.head_tiles > 1 ? 6 : 4);
+    if (prm.heads_per_wg == 1 && kv_heads > 1 && kv_heads <= 8 && prm.head_tiles == 1) {
+        prm.heads_per_wg = kv_heads;
+        prm.quarters_per_wg = 1;
+    }
+    // A grid of fewer waves than four per CU leaves CUs idle, and each busy CU
+    // can keep only so many loads in flight. The same waves then go in smaller
+    // workgroups, the largest of 4, 2 or 1 waves that still gives two
+    // workgroups per CU (else 1 wave). Measured on MI355X, Llama-3-8B geometry
+    // (decode call, us; 8 waves -> chosen): B1 L4096 12.4 -> 10.2 with 1 wave,
+    // FP8 12.6 -> 10.6-11.1, B2 L4096 and B1 L8192 13.2 -> 12.9 and 13.65 ->
+    // 13.1 with 2 waves.
     //
-    // Grids of one to two 8-wave workgroups per CU with 2, 4 or 8 KV heads and
-    // GQA groups of up to 8 take workgroups of 2 KV heads x 2 quarters instead
-    // (4 waves; quarters combined where the merge is not XCD-grouped, see the
-    // end of this function). Measured on MI355X by graph replay of 200
-    // calls, N(0,1) data, K/V sets rotated past the Infinity Cache (decode
-    // call, us): Llama-3-8B B4 L4096 18.0-18.4 -> 17.4-17.6, B8 L4096 29.45
-    // -> 28.54, B16 L4096 with 2 KV heads (GQA 8) 20.2-20.9 -> 18.5-18.8, B8
-    // L4096 with 4 KV heads 20.05 -> 19.1-19.2; ragged B4 batches within
-    // 0.1-0.25. B3 L4096 (192 workgroups) was slower with smaller workgroups
-    // of any kind (14.74 -> 15.05). Larger grids keep 8 waves when lengths
-    // are uniform (B16 L4096 55.1 -> 56.9, B32 L4096 105.7 -> 109.1) but
-    // not when they are ragged (PD_HINT_RAGGED_LENGTHS): then up to eight
-    // 8-wave workgroups per CU take the smaller ones (B16 with lengths
-    // uniform in [0, 4096] 37.8 -> 33.3, B32 65.1 -> 59.7; the reference's
-    // B16 L4096 batch 47.6 -> 44.0 in the benchmark). At sixteen per CU (a
-    // B16 page-32 L8192 batch at split 128) it was flat, so those keep 8.
-    const int64_t wg8 = shape_workgroups(prm, kv_heads);
-    if (wg8 * 2 <= cus) {  // small grid
-        const int64_t waves_total = wg8 * (partial_threads(prm) / kWave);
+    // mid_grid marks the grids of 8 to 16 waves per CU (up to 64 with ragged
+    // lengths): they stream K and V whatever their head groups, and do not
+    // fold where the merge is XCD-grouped (below).
+    const int64_t waves_total = shape_workgroups(prm, kv_heads) * (partial_threads(prm) / kWave);
+    if (waves_total <= 4ll * cus) {  // small grid
         int waves = 4;
         while (waves > 1 && waves_total / waves < 2 * cus) waves /= 2;
-        choose_workgroup(prm, kv_heads, kMfmaWorkgroupHeads, waves);
-    } else if (wg8 >= cus &&
-               item_workgroups(prm, kv_heads, prm.live_items) <= (prm.ragged_lengths ? 8 : 2) * static_cast<int64_t>(cus) &&
+        choose_workgroup(prm, kv_heads, kMfmaSmallGridHeads, waves);
+    } else if (waves_total >= 8ll * cus &&
+               item_workgroups(prm, kv_heads, prm.live_items) * (partial_threads(prm) / kWave) <=
+                   (prm.ragged_lengths ? 64ll : 16ll) * cus &&
                (kv_heads == 2 || kv_heads == 4 || kv_heads == 8) && gt <= 8) {
-        choose_workgroup(prm, kv_heads, 2, 4);
         prm.mid_grid = 1;
-    }
-    // The kernels for grids with tail items or a work list need 129-136 VGPRs
-    // (three waves per SIMD; the plain rectangular one fits 128, four): an
-    // 8-wave workgroup of theirs would hold a CU alone, so they take 4-wave
-    // workgroups. Measured on MI355X, uniform B32 L4096 with twice the
-    // context reserved and host bounds: 120.2 us per call in 8-wave
-    // workgroups; 113.2 us as a plain rectangular grid, dead partitions
-    // included. Forcing those kernels to 128 VGPRs spilled and cost more
-    // elsewhere (ragged + shared B16 40.7 -> 44.9 us).
-    if (grid_kind(prm) != kGridRect && partial_threads(prm) / kWave > 4) {
-        if ((kv_heads == 2 || kv_heads == 4 || kv_heads == 8) && gt <= 8) {
-            choose_workgroup(prm, kv_heads, 2, 4);
-            prm.mid_grid = 1;
-        } else {
-            choose_workgroup(prm, kv_heads, kMfmaWorkgroupHeads, 4);
-        }
     }
     // Combining a workgroup's quarters into one state cuts the state stores
     // (written back at the kernel's end) and the merge's reads by qw; its
@@ -1336,7 +1344,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     // 87.1, hence the conditions.
     const bool fills_device = shape_workgroups(prm, kv_heads) >= cus;
     prm.combine = fills_device && (prm.quarters_per_wg == 2 || (prm.quarters_per_wg == 4 && gt == 16));
-    const bool long_quarters = fills_device && wg8 * 2 > cus && gt <= 8 && kv_heads <= 8 && elem == 2 &&
+    const bool long_quarters = fills_device && waves_total > 4ll * cus && gt <= 8 && kv_heads <= 8 && elem == 2 &&
                                !prm.ragged_lengths && prm.split_tokens >= 1024;
     const int default_groups = kv_heads / prm.heads_per_wg;
     // When the KV heads need several workgroups (kv_heads > heads_per_wg),
@@ -1390,7 +1398,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
         prm.combine = prm.quarters_per_wg == 4;
     }
     plan_rows(prm, kv_heads, head_dim, elem, combine_slot_bytes(head_dim), mfma_stage_bytes(head_dim, elem), cus,
-              prefix_slots(prm.group));
+              prefix_slots(prm.group), row_max_waves(head_dim));
     plan_prefix_items(prm, prefix_slots(prm.group));
     plan_xcd(prm, kv_heads);
     // Where the merge reads its states from the XCD's L2 (plan_xcd), the fold
