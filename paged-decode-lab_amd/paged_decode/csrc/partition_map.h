@@ -85,6 +85,7 @@ struct PartialParams {
     int xcd_shift;
     uint32_t xcd_main_rows;
     int xcd_tail_shift;
+    int head_shift;  // plain grid: log2 of its head groups (grid_y), or -1 when they are no power of two
     // Rectangular grid (compact == 0): sequence b's partitions 0 ..
     // main_splits - 1 are items of z-slice b; when main_splits < splits (host
     // bounds reach fewer partitions than reserved), z-slices batch, batch + 1,
@@ -186,7 +187,7 @@ struct BlockCoords {
 
 template <int kList>
 PD_HD BlockCoords block_coords(uint32_t bx, uint32_t by, uint32_t bz, uint32_t gx, uint32_t gy, int xcd_shift,
-                               uint32_t xcd_main_rows, int xcd_tail_shift) {
+                               uint32_t xcd_main_rows, int xcd_tail_shift, int head_shift = -1) {
     if (xcd_shift >= 0) {
         const uint32_t x = bx & 7u;
         uint32_t r = by * 8u + x, tokens = bx >> 3;
@@ -204,6 +205,8 @@ PD_HD BlockCoords block_coords(uint32_t bx, uint32_t by, uint32_t bz, uint32_t g
     const uint64_t lin = bx + static_cast<uint64_t>(gx) * by;
     if (lin <= 0xFFFFFFFFull) {
         const uint32_t l32 = static_cast<uint32_t>(lin);
+        if (head_shift >= 0)
+            return BlockCoords{static_cast<int>(l32 >> head_shift), static_cast<int>(l32 & (gy - 1u)), static_cast<int>(bz)};
         return BlockCoords{static_cast<int>(l32 / gy), static_cast<int>(l32 % gy), static_cast<int>(bz)};
     }
     return BlockCoords{static_cast<int>(lin / gy), static_cast<int>(lin % gy), static_cast<int>(bz)};
@@ -222,16 +225,24 @@ struct PartitionRange {
     int member0, members, row;
 };
 
+// log2 of the quarters per workgroup (1, 2 or 4). The kernels' prologue, which
+// every wave runs before its first load, has no integer division on its usual
+// path: a 32-bit division by a kernel argument is some 30 dependent
+// instructions, and this one had six. Measured on MI355X (decode call, us,
+// graph): FP16 B1 L4096 9.25 -> 8.92, B2 12.3 -> 11.9, B4 17.3 -> 16.9, with
+// twice the context reserved 18.9 -> 18.2, ragged + shared B16 46.3 -> 45.7.
+PD_HD int quarter_shift(const PartialParams& p) { return p.quarters_per_wg >> 1; }
+
 inline int grid_kind(const PartialParams& prm) {
     return prm.compact ? kGridList : prm.main_splits < prm.splits ? kGridRectTails : kGridRect;
 }
 
 template <int kList>
 PD_HD PartitionRange partition_range(const PartialParams& p, const BlockCoords& bc) {
-    const int groups = kQuarters / p.quarters_per_wg;
-    const int item = bc.tokens / groups;
+    const int group_shift = 2 - quarter_shift(p);  // log2 of the quarter groups per item
+    const int item = bc.tokens >> group_shift;
     PartitionRange r;
-    r.qgroup = bc.tokens - item * groups;
+    r.qgroup = bc.tokens & ((1 << group_shift) - 1);
     r.member0 = 0;
     r.members = 1;
     if (kList == kGridRect) {
@@ -360,15 +371,20 @@ template <int GT, int ALIGN>
 PD_HD WaveWork wave_work(const PartialParams& p, int b, int split, int count, int qgroup, int heads, int wave,
                          int len_raw) {
     WaveWork w;
-    const int qw = p.quarters_per_wg;
-    const int qq = wave % qw;
-    const int tt = (wave / qw) % p.tiles_per_wg;
-    const int hh = wave / (qw * p.tiles_per_wg);
-    const int tile_groups = p.head_tiles / p.tiles_per_wg;
+    const int qs = quarter_shift(p);
+    const int qq = wave & (p.quarters_per_wg - 1);
     w.split = split;
-    w.quarter = qgroup * qw + qq;
-    w.kv_head = (heads / tile_groups) * p.heads_per_wg + hh;
-    w.tile = (heads % tile_groups) * p.tiles_per_wg + tt;
+    w.quarter = (qgroup << qs) + qq;
+    if (GT < 8 || p.head_tiles == 1) {  // a KV head's group is one tile (head_tile: always below 8)
+        w.kv_head = heads * p.heads_per_wg + (wave >> qs);
+        w.tile = 0;
+    } else {
+        const int tt = (wave >> qs) % p.tiles_per_wg;
+        const int hh = (wave >> qs) / p.tiles_per_wg;
+        const int tile_groups = p.head_tiles / p.tiles_per_wg;
+        w.kv_head = (heads / tile_groups) * p.heads_per_wg + hh;
+        w.tile = (heads % tile_groups) * p.tiles_per_wg + tt;
+    }
     const int len = imax(0, imin(len_raw, p.reach));  // decode.cu:42-44
     const int64_t first = static_cast<int64_t>(split) * p.split_tokens;
     w.dead = first >= len || count <= 0;  // count 0: an empty item of the grid
@@ -388,8 +404,7 @@ PD_HD WaveWork wave_work(const PartialParams& p, int b, int split, int count, in
 // the page-id window be requested before the sequence length arrives.
 template <int ALIGN>
 PD_HD int speculative_page(const PartialParams& p, int split, int count, int qgroup, int wave) {
-    const int qw = p.quarters_per_wg;
-    const int quarter = qgroup * qw + wave % qw;
+    const int quarter = (qgroup << quarter_shift(p)) + (wave & (p.quarters_per_wg - 1));
     const int per_full = ((count * p.split_tokens + kQuarters - 1) / kQuarters + ALIGN - 1) / ALIGN * ALIGN;
     const int capacity = p.table_width << p.page_shift;
     const int64_t start = static_cast<int64_t>(split) * p.split_tokens + static_cast<int64_t>(quarter) * per_full;
@@ -407,8 +422,8 @@ PD_HD WaveWork row_wave_work(const PartialParams& p, int b, int heads, int wave,
     WaveWork w;
     w.split = 0;
     w.quarter = wave;
-    w.kv_head = heads / p.head_tiles;
-    w.tile = heads % p.head_tiles;
+    w.kv_head = GT < 8 || p.head_tiles == 1 ? heads : heads / p.head_tiles;
+    w.tile = GT < 8 || p.head_tiles == 1 ? 0 : heads % p.head_tiles;
     const int te = imax(0, imin(len_raw, p.reach));  // decode.cu:42-44
     int per = (te + waves - 1) / waves;
     per = (per + ALIGN - 1) / ALIGN * ALIGN;
@@ -691,6 +706,16 @@ inline Grid partial_grid(const PartialParams& prm, int kv_heads) {
                                 prm.main_splits)
         : 0u;
     return Grid{static_cast<uint32_t>(prm.main_splits) * groups, heads, static_cast<uint32_t>(prm.batch) + tail_slices};
+}
+
+// The launch's grid, as the kernel's arguments carry it.
+inline void set_grid(PartialParams& prm, int kv_heads) {
+    const Grid grid = partial_grid(prm, kv_heads);
+    prm.grid_x = grid.x;
+    prm.grid_y = grid.y;
+    prm.head_shift = -1;
+    if ((grid.y & (grid.y - 1)) == 0)
+        for (prm.head_shift = 0; (1u << prm.head_shift) < grid.y;) ++prm.head_shift;
 }
 
 inline int64_t workgroups(const Grid& g) { return static_cast<int64_t>(g.x) * g.y * g.z; }
@@ -1412,9 +1437,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     // the quarters long: MQA B128 13.8 -> 15.15, uniform B32 L4096 (four
     // quarters) 88.5 -> 92.2.
     if (prm.mid_grid && prm.merge_xcd_rows > 0) prm.combine = 0;
-    const Grid grid = partial_grid(prm, kv_heads);
-    prm.grid_x = grid.x;
-    prm.grid_y = grid.y;
+    set_grid(prm, kv_heads);
 }
 
 // Launch shape of the FP32 kernel (and whole rows, as for the matrix-core
@@ -1426,9 +1449,7 @@ inline void plan_fp32(PartialParams& prm, int kv_heads, int head_dim, int cus = 
     choose_workgroup(prm, kv_heads, 8);
     plan_rows(prm, kv_heads, head_dim, 4, row_slot_bytes_fp32(head_dim), 0, cus, 1, fp32_row_max_waves(gt));
     plan_xcd(prm, kv_heads);
-    const Grid grid = partial_grid(prm, kv_heads);
-    prm.grid_x = grid.x;
-    prm.grid_y = grid.y;
+    set_grid(prm, kv_heads);
 }
 
 }  // namespace pd
