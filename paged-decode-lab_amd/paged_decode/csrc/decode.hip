@@ -31,10 +31,9 @@
 //       accumulators are rescaled only when a tile's max exceeds the running
 //       max by 2^8); each lane ends with its own slice of the state and
 //       stores it directly.
-//       partial_kernel (FP32): the same decomposition on the vector ALU;
-//       q.k is reduced over each token row's lanes with DPP, every token row
-//       keeps its own online-softmax stream, and the rows' streams are
-//       combined with lane shuffles before the store.
+//       partial_kernel (FP32): the same decomposition on the FP32 matrix ops;
+//       every row group of lanes keeps its own online-softmax stream, and the
+//       streams are combined with lane shuffles before the store.
 //     Page ids come from a 64-entry, lane-indexed window read once per wave
 //     and indexed with v_readlane; loads stream through a short register
 //     pipeline, K and V alike as whole token rows

@@ -41,13 +41,11 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 // DPP controls: quad_perm [1,0,3,2] and [2,3,0,1] swap neighbours at distance
 // 1 and 2; row_half_mirror reverses each 8-lane half-row; row_mirror reverses
 // each 16-lane row. Applied in that order, a sum/max reaches every lane of an
-// aligned 8- or 16-lane group. ds_swizzle in bit mode with xor 0x10 exchanges
-// lanes 16 apart within each 32-lane half.
+// aligned 8- or 16-lane group.
 constexpr int kDppQuadSwap1 = 0xB1;
 constexpr int kDppQuadSwap2 = 0x4E;
 constexpr int kDppRowHalfMirror = 0x141;
 constexpr int kDppRowMirror = 0x140;
-constexpr int kSwizzleSwap16 = 0x401F;
 
 template <int kCtrl>
 __device__ __forceinline__ float dpp_move(float x) {
@@ -55,20 +53,14 @@ __device__ __forceinline__ float dpp_move(float x) {
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), kCtrl, 0xF, 0xF, false));
 }
 
-__device__ __forceinline__ float swizzle_swap16(float x) {
-    return __builtin_bit_cast(float,
-                              __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), kSwizzleSwap16));
-}
-
-// Sum over each aligned group of kLanes (8, 16 or 32) lanes, result in every lane.
+// Sum over each aligned group of kLanes (8 or 16) lanes, result in every lane.
 template <int kLanes>
 __device__ __forceinline__ float group_sum(float x) {
-    static_assert(kLanes == 8 || kLanes == 16 || kLanes == 32, "unsupported group");
+    static_assert(kLanes == 8 || kLanes == 16, "unsupported group");
     x += dpp_move<kDppQuadSwap1>(x);
     x += dpp_move<kDppQuadSwap2>(x);
     x += dpp_move<kDppRowHalfMirror>(x);
     if constexpr (kLanes >= 16) x += dpp_move<kDppRowMirror>(x);
-    if constexpr (kLanes >= 32) x += swizzle_swap16(x);
     return x;
 }
 
@@ -145,29 +137,6 @@ __device__ __forceinline__ float sum_over_lane_groups(float x) {
 __device__ __forceinline__ float2 read_state(const float2* st, int j) {
     return __builtin_bit_cast(float2, reinterpret_cast<const uint64_t*>(st)[j]);
 }
-
-// ---------------------------------------------------------------------------
-// Element types of the vector-ALU kernel. A lane moves 16 bytes per load: 4 floats.
-template <typename T>
-struct Elem;
-
-template <>
-struct Elem<float> {
-    static constexpr int kPerLoad = 4;
-    static __device__ __forceinline__ float dot(const u32x4& a, const u32x4& b) {
-        const f32x4 af = __builtin_bit_cast(f32x4, a);
-        const f32x4 bf = __builtin_bit_cast(f32x4, b);
-        float acc = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc = fmaf(af[i], bf[i], acc);
-        return acc;
-    }
-    static __device__ __forceinline__ void widen(const u32x4& x, float (&f)[4]) {
-        const f32x4 v = __builtin_bit_cast(f32x4, x);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) f[i] = v[i];
-    }
-};
 
 }  // namespace pd
 

@@ -60,29 +60,86 @@ __device__ __forceinline__ void store_empty_states(const PartialParams& p, const
 }
 
 // ---------------------------------------------------------------------------
-// FP32 (and generic) partition kernel, VALU only.
+// FP32 partition kernel: both contractions on v_mfma_f32_4x4x1_16b_f32, whose
+// products and sums are those of fmaf.
 //
-// Lanes [r*LPT, (r+1)*LPT) hold token r of a TPL-token load (16 bytes each);
-// q.k is a per-lane partial dot reduced over the LPT lanes of the row with DPP;
-// every token row keeps its own online-softmax stream, combined across rows at
-// the end of the wave. Chunks of NL loads stream through PD + 1 register
-// buffers in fully unrolled blocks of NC chunks.
+// A wave takes tiles of four tokens. K is loaded as lane (block = lane / 4,
+// token = lane % 4), 16 bytes per lane: the MFMA's rows are the tile's tokens,
+// its columns four query heads and its sixteen blocks sixteen slices of the
+// dims, so each lane ends with four tokens' partial scores of head lane % 4.
+// Summing them over the blocks also spreads the tokens (sum_scores): row group
+// r of the lanes -- [r*LPT, (r+1)*LPT) -- keeps tokens r, r + TPL, ..., which is
+// the A operand of P.V (rows = heads, blocks = dims), V being loaded in row
+// layout: lanes of row group r hold token r of a TPL-token load, 16 bytes each.
+// Every row group keeps its own online-softmax stream, head h's in the lanes
+// with lane % 4 == h % 4; they are combined at the end of the wave.
+//
+// Per four FP32 tokens of D 128 with four heads: 16 MFMAs (8 cycles each) and
+// about 45 other vector instructions. The vector ALU alone took about 200, with
+// a 5-step sum over the lanes for each head and token and a softmax that every
+// lane repeated, and waited for its loads at the end of each block of 32 tokens.
+// A ring of R tiles stays in flight: the next K is requested once a tile is
+// scored, the next V once it is summed. Measured on
+// MI355X (decode call, us, with the launch shape of plan_fp32; vector ALU ->
+// this): B8 L4096 ragged, 158 MB 44.68 -> 35.66; uniform B2 L4096 23.96 ->
+// 16.11, B16 116.93 -> 101.95;
+// MHA B1 L16384 106.71 -> 88.46; D 64: GQA 8 B32 L3000 ragged 53.66 -> 34.95, MQA B64
+// L2048 39.40 -> 25.06; whole rows B64 L256 35.18 -> 28.33.
 // kRow: a whole-row workgroup (up to kRowMaxWaves waves) that folds its
 // waves' states in LDS and writes the output rows instead of states.
-template <typename T, int D, int GT, int NL, int PD, int NC, int kList, bool kRow = false>
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const char* base, uint32_t bytes);
+
+// Sums of a 4-token score quadruple over the MFMA's blocks (lanes lane % 4
+// apart): x[s] is token TPL * s + lane / LPT of the tile, in all lanes of its
+// row group with the same lane % 4.
+template <int LPT>
+__device__ __forceinline__ void sum_scores(const f32x4& sc, float (&x)[LPT / 16]) {
+    constexpr int kRowRor4 = 0x124, kRowRor8 = 0x128;
+    if constexpr (LPT == 32) {
+        x[0] = swap32_sum(sc[0], sc[1]);
+        x[1] = swap32_sum(sc[2], sc[3]);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) x[s] = swap16_sum(x[s], x[s]);
+    } else {
+        const float even = swap32_sum(sc[0], sc[2]), odd = swap32_sum(sc[1], sc[3]);
+        x[0] = swap16_sum(even, odd);
+    }
+#pragma unroll
+    for (int s = 0; s < LPT / 16; ++s) {
+        x[s] += dpp_move<kRowRor4>(x[s]);
+        x[s] += dpp_move<kRowRor8>(x[s]);
+    }
+}
+
+// Lane 4 * (lane / 4) + kLane's value.
+template <int kLane>
+__device__ __forceinline__ float quad_lane(float x) {
+    return dpp_move<kLane * 0x55>(x);
+}
+
+__device__ __forceinline__ float quad_lane(float x, int i) {
+    return i == 0 ? quad_lane<0>(x) : i == 1 ? quad_lane<1>(x) : i == 2 ? quad_lane<2>(x) : quad_lane<3>(x);
+}
+
+template <int D, int GT, int R, bool kStreamV, int kList, bool kRow = false>
 __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave * 8)
     partial_kernel(const PartialParams p) {
-    using E = Elem<T>;
-    constexpr int EPL = E::kPerLoad;
+    constexpr int EPL = 4;
     constexpr int LPT = D / EPL;
     constexpr int TPL = kWave / LPT;
-    constexpr int CT = NL * TPL;
-    static_assert(TPL >= 2 && TPL <= 8 && (TPL & (TPL - 1)) == 0, "unsupported row split");
+    constexpr int TT = kFp32TileTokens;
+    constexpr int NL = TT / TPL;        // loads per tile of K, and of V
+    constexpr int HG = (GT + 3) / 4;    // head groups of four
+    static_assert(D == 64 * NL, "K loads of 64 dims");
 
-    struct Chunk {
+    struct Tile {
         u32x4 k[NL];
         u32x4 v[NL];
-        uint32_t live;
+    };
+    struct Request {
+        uint64_t base;
+        uint32_t bytes;  // of the tile's live rows (0: nothing to read)
     };
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -94,12 +151,12 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
     const PartitionRange pr = partition_range<kList>(p, bc);
     const int waves_wg = blockDim.x / kWave;
     const int32_t* pages = p.table + static_cast<int64_t>(pr.b) * p.table_width;
-    int window = kRow ? row_speculative_page<TPL>(p, wave, waves_wg)
-                      : speculative_page<TPL>(p, pr.first, pr.count, pr.qgroup, wave);
+    int window = kRow ? row_speculative_page<TT>(p, wave, waves_wg)
+                      : speculative_page<TT>(p, pr.first, pr.count, pr.qgroup, wave);
     int window_ids = pages[window_entry(p, window, lane)];
     const int len_raw = p.lengths[pr.b];
-    const WaveWork w = kRow ? row_wave_work<GT, TPL>(p, pr.b, bc.heads, wave, waves_wg, len_raw)
-                            : wave_work<GT, TPL>(p, pr.b, pr.first, pr.count, pr.qgroup, bc.heads, wave, len_raw);
+    const WaveWork w = kRow ? row_wave_work<GT, TT>(p, pr.b, bc.heads, wave, waves_wg, len_raw)
+                            : wave_work<GT, TT>(p, pr.b, pr.first, pr.count, pr.qgroup, bc.heads, wave, len_raw);
     // Whole-row waves with an empty slice stay for the fold (empty state).
     if (!kRow && w.dead) {
         // Never read: the merge stops at the sequence's last live partition.
@@ -109,106 +166,117 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
         asm volatile("" ::"v"(window_ids));
         return;
     }
-    const T* q_base = static_cast<const T*>(p.q) + w.q_row * D;
+    const float* q_base = static_cast<const float*>(p.q) + w.q_row * D;
 
-    u32x4 qv[GT];
+    // B operand of q.K^T: head 4 hg + lane % 4, dims 64 i + 4 (lane / 4) on.
+    f32x4 qv[HG][NL];
 #pragma unroll
-    for (int g = 0; g < GT; ++g) {
-        qv[g] = u32x4{0u, 0u, 0u, 0u};
-        if (g < w.heads_here) qv[g] = *reinterpret_cast<const u32x4*>(q_base + g * D + col * EPL);
-    }
-    float m[GT], l[GT], acc[GT][EPL];
-#pragma unroll
-    for (int g = 0; g < GT; ++g) {
-        m[g] = kNoToken;
-        l[g] = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
-    }
-    const char* k_head = static_cast<const char*>(p.k) + static_cast<size_t>(w.kv_head) * D * sizeof(T);
-    const char* v_head = static_cast<const char*>(p.v) + static_cast<size_t>(w.kv_head) * D * sizeof(T);
-    // Groups with no live token are redirected to this tile's q row: always
-    // mapped, finite, and the same line for every lane.
-    const char* park = reinterpret_cast<const char*>(q_base);
-    const uint32_t lane_bytes = static_cast<uint32_t>(col) * 16u;
-    int rb = w.wb, re = w.wb;
-
-    auto issue = [&](Chunk& ch, int c0, int ids, int win) {
-        const char* kp[NL];
-        const char* vp[NL];
-        uint32_t off[NL];
-        uint32_t live = 0;
+    for (int hg = 0; hg < HG; ++hg) {
+        const int head = 4 * hg + lane % 4;
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            const int g = c0 + i * TPL;
-            const TileSpan span = tile_span(p, g, TPL, rb, re, win);
-            const int page = __builtin_amdgcn_readlane(ids, span.slot);
-            const bool ok = tile_live(p, g, re, page);
-            live |= static_cast<uint32_t>(ok) << i;
-            const uint64_t page_off = tile_page_offset(p, ok, page);
-            kp[i] = ok ? k_head + page_off : park;
-            vp[i] = ok ? v_head + page_off : park;
-            off[i] = token_offset(p, ok, g + row, span, lane_bytes);
+            qv[hg][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (head < w.heads_here)
+                qv[hg][i] = *reinterpret_cast<const f32x4*>(q_base + head * D + 64 * i + 4 * (lane / 4));
         }
-        ch.live = live;
+    }
+    float m_head[HG], l_head[HG];  // of head 4 hg + lane % 4 and this lane's row group
+    f32x4 sum[HG][EPL];            // sum[hg][e][r]: head 4 hg + r, dim col * EPL + e
 #pragma unroll
-        for (int i = 0; i < NL; ++i) ch.k[i] = *reinterpret_cast<const u32x4*>(kp[i] + off[i]);
+    for (int hg = 0; hg < HG; ++hg) {
+        m_head[hg] = kNoToken;
+        l_head[hg] = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) ch.v[i] = *reinterpret_cast<const u32x4*>(vp[i] + off[i]);
+        for (int e = 0; e < EPL; ++e) sum[hg][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const char* k_head = static_cast<const char*>(p.k) + static_cast<size_t>(w.kv_head) * D * 4;
+    const char* v_head = static_cast<const char*>(p.v) + static_cast<size_t>(w.kv_head) * D * 4;
+    const uint32_t k_lane = tile_row_offset(p, lane % 4, static_cast<uint32_t>(lane / 4) * 16u);
+    const uint32_t v_lane = tile_row_offset(p, row, static_cast<uint32_t>(col) * 16u);
+    int rb = w.wb, re = w.wb;
+
+    auto locate = [&](int t0) {
+        const int page = __builtin_amdgcn_readlane(window_ids, tile_slot(p, t0, window));
+        return Request{tile_base(p, page, t0), tile_bytes(p, tile_live(p, t0, re, page), t0, re, TT)};
+    };
+    auto load_k = [&](Tile& t, const Request& rq) {
+        const __amdgpu_buffer_rsrc_t kb = tile_buffer(k_head + rq.base, rq.bytes);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) t.k[i] = __builtin_amdgcn_raw_buffer_load_b128(kb, k_lane + 256u * i, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_v = [&](Tile& t, const Request& rq) {
+        const __amdgpu_buffer_rsrc_t vb = tile_buffer(v_head + rq.base, rq.bytes);
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            t.v[i] = __builtin_amdgcn_raw_buffer_load_b128(vb, v_lane + tile_row_offset(p, TPL * i, 0), 0,
+                                                           kStreamV ? 2 : 0);
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    auto consume = [&](const Chunk& ch, int c0) {
-        float s[NL][GT];
+    auto score = [&](const Tile& t, float (&x)[HG][NL]) {
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int t = c0 + i * TPL + row;
-            const bool valid = (((ch.live >> i) & 1u) != 0u) & (t >= rb) & (t < re);
+        for (int hg = 0; hg < HG; ++hg) {
+            f32x4 sc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int g = 0; g < GT; ++g) {
-                const float d = group_sum<LPT>(E::dot(qv[g], ch.k[i]));
-                s[i][g] = valid ? d : -INFINITY;
+            for (int i = 0; i < NL; ++i) {
+                const f32x4 kf = __builtin_bit_cast(f32x4, t.k[i]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sc = __builtin_amdgcn_mfma_f32_4x4x1f32(kf[e], qv[hg][i][e], sc, 0, 0, 0);
+            }
+            sum_scores<LPT>(sc, x[hg]);
+        }
+    };
+
+    auto accumulate = [&](Tile& t, const Request& rq, float (&x)[HG][NL], int t0) {
+        if (rq.bytes == 0u || t0 < rb || t0 + TT > re) {
+#pragma unroll
+            for (int s = 0; s < NL; ++s) {
+                const int token = t0 + TPL * s + row;
+                const bool valid = (rq.bytes != 0u) & (token >= rb) & (token < re);
+#pragma unroll
+                for (int hg = 0; hg < HG; ++hg) x[hg][s] = valid ? x[hg][s] : -INFINITY;
+                // Rows before the range are another quarter's: their V stays out of this one's sums.
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t.v[s][e] = token >= rb ? t.v[s][e] : 0u;
             }
         }
-        float chunk_max[GT];
+        float top[HG];
         bool grow = false;
 #pragma unroll
-        for (int g = 0; g < GT; ++g) {
-            float cm = s[0][g];
+        for (int hg = 0; hg < HG; ++hg) {
+            top[hg] = x[hg][0];
 #pragma unroll
-            for (int i = 1; i < NL; ++i) cm = fmaxf(cm, s[i][g]);
-            chunk_max[g] = cm * p.scale_log2;
-            grow |= chunk_max[g] > m[g] + kRescaleSlack;
+            for (int s = 1; s < NL; ++s) top[hg] = fmaxf(top[hg], x[hg][s]);
+            top[hg] *= p.scale_log2;
+            grow |= top[hg] > m_head[hg] + kRescaleSlack;
         }
         if (__any(grow)) {
 #pragma unroll
-            for (int g = 0; g < GT; ++g) {
-                const float m_new = fmaxf(m[g], chunk_max[g]);
-                const float alpha = fast_exp2(m[g] - m_new);
-                m[g] = m_new;
-                l[g] *= alpha;
+            for (int hg = 0; hg < HG; ++hg) {
+                const float m_new = fmaxf(m_head[hg], top[hg]);
+                const float alpha = fast_exp2(m_head[hg] - m_new);
+                m_head[hg] = m_new;
+                l_head[hg] *= alpha;
 #pragma unroll
-                for (int e = 0; e < EPL; ++e) acc[g][e] *= alpha;
+                for (int r = 0; r < 4; ++r) {
+                    const float a = quad_lane(alpha, r);
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) sum[hg][e][r] *= a;
+                }
             }
         }
 #pragma unroll
-        for (int g = 0; g < GT; ++g) {
-            float sum = l[g];
+        for (int hg = 0; hg < HG; ++hg) {
 #pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                s[i][g] = fast_exp2(fmaf(s[i][g], p.scale_log2, -m[g]));
-                sum += s[i][g];
+            for (int s = 0; s < NL; ++s) {
+                const float wt = fast_exp2(fmaf(x[hg][s], p.scale_log2, -m_head[hg]));
+                l_head[hg] += wt;
+                const f32x4 vf = __builtin_bit_cast(f32x4, t.v[s]);
+#pragma unroll
+                for (int e = 0; e < EPL; ++e)
+                    sum[hg][e] = __builtin_amdgcn_mfma_f32_4x4x1f32(wt, vf[e], sum[hg][e], 0, 0, 0);
             }
-            l[g] = sum;
-        }
-#pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            float vf[EPL];
-            E::widen(ch.v[i], vf);
-#pragma unroll
-            for (int g = 0; g < GT; ++g)
-#pragma unroll
-                for (int e = 0; e < EPL; ++e) acc[g][e] = fmaf(s[i][g], vf[e], acc[g][e]);
         }
     };
 
@@ -218,19 +286,38 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
             window_ids = pages[window_entry(p, window, lane)];
         }
         re = min(w.we, (window + kWave) << p.page_shift);
-        for (int s0 = rb & ~(TPL - 1); s0 < re; s0 += NC * CT) {
-            Chunk buf[PD + 1];
+        Tile ring[R];
+        Request at[R];
+        int s0 = rb & ~(TT - 1);
 #pragma unroll
-            for (int n = 0; n < PD; ++n) issue(buf[n], s0 + n * CT, window_ids, window);
+        for (int c = 0; c < R; ++c) {
+            at[c] = locate(s0 + c * TT);
+            load_k(ring[c], at[c]);
+            load_v(ring[c], at[c]);
+        }
+        for (; s0 < re; s0 += R * TT) {
 #pragma unroll
-            for (int n = 0; n < NC; ++n) {
-                if (s0 + n * CT >= re) break;
-                if (n + PD < NC) issue(buf[(n + PD) % (PD + 1)], s0 + (n + PD) * CT, window_ids, window);
-                consume(buf[n % (PD + 1)], s0 + n * CT);
+            for (int c = 0; c < R; ++c) {
+                float x[HG][NL];
+                score(ring[c], x);
+                const Request next = locate(s0 + (R + c) * TT);
+                load_k(ring[c], next);
+                accumulate(ring[c], at[c], x, s0 + c * TT);
+                load_v(ring[c], next);
+                at[c] = next;
             }
         }
     }
 
+    // The row group's state with every head in every lane.
+    float m[GT], l[GT], acc[GT][EPL];
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+        m[g] = quad_lane(m_head[g / 4], g % 4);
+        l[g] = quad_lane(l_head[g / 4], g % 4);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[g][e] = sum[g / 4][e][g % 4];
+    }
     // Combine the TPL token-row streams (lanes LPT, 2*LPT, ... apart).
 #pragma unroll
     for (int g = 0; g < GT; ++g) {
@@ -937,14 +1024,6 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? PD_OK : PD_ERR_LAUNCH; }
 
-// FP32 kernel: 16-byte loads of K (and of V) per lane per chunk, chunks in
-// flight ahead of the one being consumed, chunks per straight-line block.
-constexpr int kFp32ChunkLoads = 1;
-constexpr int kFp32Prefetch = 4;
-constexpr int kFp32BlockChunks = 16;
-// Whole-row FP32 launches give each wave a slice of a few chunks (16 tokens
-// at most rows' sizes): a block of four keeps the straight-line code short.
-constexpr int kFp32RowBlockChunks = 4;
 // Matrix-core kernel: pairs of 16-token tiles in flight per wave.
 constexpr int kMfmaRing = 1;
 
@@ -1012,17 +1091,25 @@ template <int D, int GT>
 int launch_fp32(const PartialParams& prm, int kv_heads, hipStream_t stream) {
     const dim3 grid = to_dim3(partial_grid(prm, kv_heads));
     const dim3 block(partial_threads(prm));
-    constexpr int NL = kFp32ChunkLoads, PD = kFp32Prefetch, NC = kFp32BlockChunks;
     const int kind = grid_kind(prm);
+#define PD_LAUNCH_FP32(STREAM)                                                                                      \
+    do {                                                                                                            \
+        if (kind == kGridList)                                                                                      \
+            hipLaunchKernelGGL((partial_kernel<D, GT, kFp32Ring, STREAM, kGridList>), grid, block, 0, stream, prm); \
+        else if (kind == kGridRectTails)                                                                            \
+            hipLaunchKernelGGL((partial_kernel<D, GT, kFp32Ring, STREAM, kGridRectTails>), grid, block, 0, stream,  \
+                               prm);                                                                                \
+        else                                                                                                        \
+            hipLaunchKernelGGL((partial_kernel<D, GT, kFp32Ring, STREAM, kGridRect>), grid, block, 0, stream, prm); \
+    } while (0)
     if (prm.row_mode)
-        hipLaunchKernelGGL((partial_kernel<float, D, GT, NL, PD, kFp32RowBlockChunks, kGridRect, true>), grid, block,
+        hipLaunchKernelGGL((partial_kernel<D, GT, kFp32RowRing, false, kGridRect, true>), grid, block,
                            static_cast<size_t>(prm.row_waves) * row_slot_bytes_fp32(D), stream, prm);
-    else if (kind == kGridList)
-        hipLaunchKernelGGL((partial_kernel<float, D, GT, NL, PD, NC, kGridList>), grid, block, 0, stream, prm);
-    else if (kind == kGridRectTails)
-        hipLaunchKernelGGL((partial_kernel<float, D, GT, NL, PD, NC, kGridRectTails>), grid, block, 0, stream, prm);
+    else if (prm.stream_mode != 0)
+        PD_LAUNCH_FP32(true);
     else
-        hipLaunchKernelGGL((partial_kernel<float, D, GT, NL, PD, NC, kGridRect>), grid, block, 0, stream, prm);
+        PD_LAUNCH_FP32(false);
+#undef PD_LAUNCH_FP32
     return launch_status();
 }
 

@@ -27,6 +27,9 @@ namespace pd {
 constexpr int kWave = 64;
 constexpr int kQuarters = 4;     // states per partition (quarters of the partition)
 constexpr int kTileTokens = 16;  // tokens per matrix-core tile
+constexpr int kFp32TileTokens = 4;  // and per tile of the FP32 kernel: one MFMA's rows
+constexpr int kFp32Ring = 2;        // FP32 tiles in flight per wave
+constexpr int kFp32RowRing = 4;     // and of a whole-row wave, whose slice is few tiles
 constexpr int kMi355xCus = 256;  // compute units of an MI355X
 
 // Compacted work lists are passed in the kernel arguments for batches of up
@@ -450,42 +453,13 @@ PD_HD int window_entry(const PartialParams& p, int window, int lane) {
     return imin(window + lane, p.table_width - 1);
 }
 
-// One load group of `tokens` tokens starting at t0 (a 16-token matrix-core
-// tile, or one token row group of the FP32 kernel) within the wave's current
-// range [rb, re): the live token span [lo, hi] (or the last live token when
-// the group lies past re) and the page-id window slot of its first token.
-struct TileSpan {
-    int lo, hi, slot;
-};
-
-PD_HD TileSpan tile_span(const PartialParams& p, int t0, int tokens, int rb, int re, int window) {
-    TileSpan s;
-    s.lo = imax(t0, rb);
-    s.hi = imin(t0 + tokens, re) - 1;
-    if (s.lo > s.hi) s.lo = s.hi = re - 1;
-    s.slot = imin(imax((s.lo >> p.page_shift) - window, 0), kWave - 1);
-    return s;
-}
-
-// Whether the group's loads go to its page (else to the park row: a group
-// past re, or a page id outside [0, physical_pages), decode.cu:56-58).
+// Whether the tile at t0 of a range that ends at re is read: not past re, nor
+// from a page id outside [0, physical_pages) (decode.cu:56-58).
 PD_HD bool tile_live(const PartialParams& p, int t0, int re, int page) {
     return t0 < re && static_cast<uint32_t>(page) < static_cast<uint32_t>(p.physical_pages);
 }
 
-// Byte offset of a live group's page from the head's base: page * page_bytes.
-PD_HD uint64_t tile_page_offset(const PartialParams& p, bool ok, int page) {
-    return static_cast<uint64_t>(ok ? page : 0) * p.page_bytes;
-}
-
-// Byte offset within the page (or the park row) of token t, clamped into
-// [lo, hi], at lane byte offset lane_bytes of the token's head slice.
-PD_HD uint32_t token_offset(const PartialParams& p, bool ok, int t, const TileSpan& s, uint32_t lane_bytes) {
-    const int tk = imin(imax(t, s.lo), s.hi);
-    return ok ? static_cast<uint32_t>(tk & ((1 << p.page_shift) - 1)) * p.token_bytes + lane_bytes : lane_bytes;
-}
-
-// The matrix-core kernel reads a tile through a buffer descriptor: base
+// The kernels read a tile (16 tokens, FP32: 4) through a buffer descriptor: base
 // tile_base bytes from the head's first page (the tile's first token, which a
 // tile never leaves the page of), tile_bytes long, row i of the tile at
 // tile_row_offset(i). Rows from the range's end re on, and every row of a tile
@@ -499,8 +473,8 @@ PD_HD uint64_t tile_base(const PartialParams& p, int page, int t0) {
     return static_cast<uint64_t>(static_cast<uint32_t>(page)) * static_cast<uint32_t>(p.page_bytes) +
            static_cast<uint32_t>(t0 & ((1 << p.page_shift) - 1)) * p.token_bytes;
 }
-PD_HD uint32_t tile_bytes(const PartialParams& p, bool ok, int t0, int re) {
-    return ok ? static_cast<uint32_t>(imin(kTileTokens, re - t0)) * p.token_bytes : 0u;
+PD_HD uint32_t tile_bytes(const PartialParams& p, bool ok, int t0, int re, int tokens = kTileTokens) {
+    return ok ? static_cast<uint32_t>(imin(tokens, re - t0)) * p.token_bytes : 0u;
 }
 PD_HD uint32_t tile_row_offset(const PartialParams& p, int row, uint32_t lane_bytes) {
     return static_cast<uint32_t>(row) * p.token_bytes + lane_bytes;
@@ -1446,7 +1420,17 @@ inline void plan_fp32(PartialParams& prm, int kv_heads, int head_dim, int cus = 
     const int gt = head_tile(prm.group, 8);
     prm.head_tile = gt;
     prm.head_tiles = (prm.group + gt - 1) / gt;
-    choose_workgroup(prm, kv_heads, 8);
+    // Workgroups of 4 waves over up to 4 KV heads, V streamed past the caches
+    // where no pages are shared. K is not: a lane quad reads 16 bytes of four
+    // token rows, so its cache lines are asked for twice. Measured on
+    // MI355X (decode call, us): nothing / V / K and V streamed, ring of four,
+    // 8 waves: B8 L4096 ragged 45.0 / 35.8 / 39.9; 25-50% shared pages,
+    // nothing / V: 28.5 / 30.3. Over 8 heads in 8 waves / 4 in 4 (V streamed,
+    // ring of four): B16 L4096 113.5 / 101.9, B2 19.2 / 16.5, MHA B1 L16384
+    // 93.2 / 87.6, B32 L3000 with 4 heads of D 64 39.7 / 34.7. Ring of four /
+    // two (8 waves): B16 L4096 113.5 / 107.5, B8 ragged 35.7 / 34.5.
+    choose_workgroup(prm, kv_heads, 4, 4);
+    prm.stream_mode = prm.unshared_pages ? 1 : 0;
     plan_rows(prm, kv_heads, head_dim, 4, row_slot_bytes_fp32(head_dim), 0, cus, 1, fp32_row_max_waves(gt));
     plan_xcd(prm, kv_heads);
     set_grid(prm, kv_heads);

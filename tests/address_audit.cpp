@@ -5,14 +5,13 @@
 // code (partition_map.h: plan_items, plan_mfma / plan_fp32, partial_grid) and
 // then every workgroup, wave, lane and load group of the grid is walked with
 // the same device-side functions the kernels call (block_coords,
-// partition_range, wave_work, speculative_page, window_entry, tile_span,
-// tile_live, tile_page_offset, token_offset, numerator_offset, stats_offset),
-// following the kernels' loop structure (page-id windows of 64 entries, load
-// groups issued two ahead in blocks of two for the matrix-core kernel -- four
-// and four with FP8 K/V outside whole rows -- and four ahead in blocks of sixteen for the FP32
-// kernel). Every global load is
-// checked to lie inside q, k, v, table or lengths (parked loads of dead
-// groups inside q), every store inside numerator or stats, every LDS access
+// partition_range, wave_work, speculative_page, window_entry, tile_slot,
+// tile_live, tile_base, tile_bytes, tile_row_offset, numerator_offset,
+// stats_offset), following the kernels' loop structure (page-id windows of 64
+// entries, a ring of two 16-token tiles for the matrix-core kernel and of
+// kFp32Ring or kFp32RowRing 4-token ones for the FP32 kernel, each requested again one ring on).
+// Every global load that its buffer descriptor lets through is
+// checked to lie inside q, k, v, table or lengths, every store inside numerator or stats, every LDS access
 // inside the launch's dynamic LDS; every live token is read from the page its
 // table entry names; and every live state slot is written exactly once, none
 // past a sequence's end. Built with -fsanitize=address,undefined by
@@ -198,47 +197,54 @@ int page_of(const Problem& pr, int b, int window, int slot, const PartialParams&
     return pr.table[static_cast<size_t>(b) * pr.width + entry];
 }
 
-// One load group of the matrix-core kernel (a 16-token tile), all 64 lanes.
+// The page id read for the tile of `tokens` tokens at t0. Where the tile is
+// live it is the table entry of the tile's logical page, and the tile's live
+// tokens lie on that one page, inside the sequence.
+int tile_page(const Problem& pr, const PartialParams& p, int b, int t0, int tokens, int rb, int re, int window,
+              int len) {
+    const int slot = tile_slot(p, t0, window);
+    AUDIT(slot >= 0 && slot < kWave, "window slot %d", slot);
+    const int page = page_of(pr, b, window, slot, p);
+    if (tile_live(p, t0, re, page)) {
+        const int lo = imax(t0, rb), hi = imin(t0 + tokens, re) - 1;
+        AUDIT((lo >> p.page_shift) == window + slot, "tile %d reads window slot %d of window %d", t0, slot, window);
+        AUDIT(hi >> p.page_shift == t0 >> p.page_shift, "tile %d straddles a page", t0);
+        AUDIT(lo <= hi && hi < len, "tile %d span [%d, %d] outside [%d, %d)", t0, lo, hi, rb, re);
+    }
+    return page;
+}
+
+// One tile of the matrix-core kernel (16 tokens), all 64 lanes.
 template <int D>
 void mfma_tile(const Problem& pr, const PartialParams& p, const Buffers& buf, const WaveWork& w, int b, int t0,
                int rb, int re, int window, int wave, int waves, int len, const std::vector<int>& members) {
     const int ES = pr.kv_elem;
     const int VH = D / 16, VW = VH * ES / 4, KR = D * ES / 16, TK = kWave / KR, KL = kTileTokens / TK;
     const int stage_row = mfma_stage_bytes(D, ES) / kTileTokens;
-    const TileSpan span = tile_span(p, t0, kTileTokens, rb, re, window);
-    AUDIT(span.slot >= 0 && span.slot < kWave, "window slot %d", span.slot);
-    const int page = page_of(pr, b, window, span.slot, p);
+    const int page = tile_page(pr, p, b, t0, kTileTokens, rb, re, window, len);
     const bool ok = tile_live(p, t0, re, page);
     if (ok) {
-        // The page id read is the table entry of the tile's logical page, and
-        // the tile's live tokens lie on that one page, inside the sequence.
-        AUDIT((span.lo >> p.page_shift) == window + span.slot, "tile %d reads window slot %d of window %d", t0,
-              span.slot, window);
-        AUDIT((span.hi >> p.page_shift) == (span.lo >> p.page_shift), "tile %d straddles a page", t0);
-        AUDIT(span.lo >= rb && span.hi < re && span.hi < len, "tile %d span [%d, %d] outside [%d, %d)", t0, span.lo,
-              span.hi, rb, re);
+        const int lo = imax(t0, rb);
         // A shared-prefix item reads its leader's page for its members: every
         // reader with live tokens in the tile must name that page.
         {
-            const int logical = span.lo >> p.page_shift;
+            const int logical = lo >> p.page_shift;
             for (int s : members) {
                 const int member_len = imax(0, imin(pr.lengths[s], reach_of(pr)));
-                if (span.lo < member_len)
+                if (lo < member_len)
                     AUDIT(pr.table[static_cast<size_t>(s) * pr.width + logical] == page,
                           "tile %d: member %d maps page %d, the item reads page %d", t0, s,
                           pr.table[static_cast<size_t>(s) * pr.width + logical], page);
             }
         }
     }
-    const uint64_t page_off = tile_page_offset(p, ok, page);
-    const uint64_t head_off = static_cast<uint64_t>(w.kv_head) * D * ES;
-    const uint64_t park = static_cast<uint64_t>(w.q_row) * D * 2;
+    const uint64_t base = static_cast<uint64_t>(w.kv_head) * D * ES + (ok ? tile_base(p, page, t0) : 0);
+    const uint32_t bytes = tile_bytes(p, ok, t0, re);
     for (int lane = 0; lane < kWave; ++lane) {
         const int n = lane % 16, g = lane / 16;
         for (int s = 0; s < KL; ++s) {
-            const uint32_t off = token_offset(p, ok, t0 + TK * s + lane / KR, span, static_cast<uint32_t>(lane % KR) * 16u);
-            if (ok) AUDIT(head_off + page_off + off + 16 <= buf.kv_bytes, "K load past the cache");
-            else AUDIT(park + off + 16 <= buf.q_bytes, "parked K load past q");
+            const uint32_t off = tile_row_offset(p, TK * s + lane / KR, static_cast<uint32_t>(lane % KR) * 16u);
+            if (off < bytes) AUDIT(base + off + 16 <= buf.kv_bytes, "K load past the cache");
             const int lds = wave * kTileTokens * stage_row + (TK * s + lane / KR) * stage_row + (lane % KR) * 16;
             AUDIT(lds >= 0 && lds + (ES == 2 ? 16 : 8) <= waves * mfma_stage_bytes(D, ES), "K stage write");
         }
@@ -247,33 +253,38 @@ void mfma_tile(const Problem& pr, const PartialParams& p, const Buffers& buf, co
             AUDIT(lds + (ES == 2 ? 16 : 8) <= (wave + 1) * mfma_stage_bytes(D, ES), "K stage read outside the wave's tile");
         }
         for (int e = 0; e < 4; ++e) {
-            const uint32_t off = token_offset(p, ok, t0 + 4 * e + g, span, static_cast<uint32_t>(n) * VH * ES);
-            if (ok) AUDIT(head_off + page_off + off + 4u * VW <= buf.kv_bytes, "V load past the cache");
-            else AUDIT(park + off + 4u * VW <= buf.q_bytes, "parked V load past q");
+            const uint32_t off = tile_row_offset(p, 4 * e + g, static_cast<uint32_t>(n) * VH * ES);
+            if (off < bytes) AUDIT(base + off + 4u * VW <= buf.kv_bytes, "V load past the cache");
         }
     }
 }
 
-// One load group of the FP32 kernel (TPL tokens, NL = 1 load per chunk).
+// One tile of the FP32 kernel (kFp32TileTokens tokens), all 64 lanes: K by
+// token lane % 4, V by token rows of D / 4 lanes.
 template <int D>
-void fp32_group(const Problem& pr, const PartialParams& p, const Buffers& buf, const WaveWork& w, int b, int g0,
-                int rb, int re, int window, int len) {
+void fp32_tile(const Problem& pr, const PartialParams& p, const Buffers& buf, const WaveWork& w, int b, int t0,
+               int rb, int re, int window, int len) {
     const int LPT = D / 4, TPL = kWave / LPT;
-    const TileSpan span = tile_span(p, g0, TPL, rb, re, window);
-    const int page = page_of(pr, b, window, span.slot, p);
-    const bool ok = tile_live(p, g0, re, page);
-    if (ok) {
-        AUDIT((span.lo >> p.page_shift) == window + span.slot, "group %d reads the wrong window slot", g0);
-        AUDIT((span.hi >> p.page_shift) == (span.lo >> p.page_shift), "group %d straddles a page", g0);
-        AUDIT(span.lo >= rb && span.hi < re && span.hi < len, "group %d span outside the range", g0);
-    }
-    const uint64_t page_off = tile_page_offset(p, ok, page);
-    const uint64_t head_off = static_cast<uint64_t>(w.kv_head) * D * 4;
-    const uint64_t park = static_cast<uint64_t>(w.q_row) * D * 4;
+    const int page = tile_page(pr, p, b, t0, kFp32TileTokens, rb, re, window, len);
+    const bool ok = tile_live(p, t0, re, page);
+    const uint64_t base = static_cast<uint64_t>(w.kv_head) * D * 4 + (ok ? tile_base(p, page, t0) : 0);
+    const uint32_t bytes = tile_bytes(p, ok, t0, re, kFp32TileTokens);
     for (int lane = 0; lane < kWave; ++lane) {
-        const uint32_t off = token_offset(p, ok, g0 + lane / LPT, span, static_cast<uint32_t>(lane % LPT) * 16u);
-        if (ok) AUDIT(head_off + page_off + off + 16 <= buf.kv_bytes, "K/V load past the cache");
-        else AUDIT(park + off + 16 <= buf.q_bytes, "parked load past q");
+        const uint32_t k_lane = tile_row_offset(p, lane % 4, static_cast<uint32_t>(lane / 4) * 16u);
+        const uint32_t v_lane = tile_row_offset(p, lane / LPT, static_cast<uint32_t>(lane % LPT) * 16u);
+        for (int i = 0; i < kFp32TileTokens / TPL; ++i) {
+            const uint32_t k = k_lane + 256u * i, v = v_lane + tile_row_offset(p, TPL * i, 0);
+            if (k < bytes) {
+                AUDIT(base + k + 16 <= buf.kv_bytes, "K load past the cache");
+                AUDIT(k % p.token_bytes + 16 <= D * 4u && t0 + static_cast<int>(k / p.token_bytes) < re,
+                      "K load of another head or past the range");
+            }
+            if (v < bytes) {
+                AUDIT(base + v + 16 <= buf.kv_bytes, "V load past the cache");
+                AUDIT(v % p.token_bytes + 16 <= D * 4u && t0 + static_cast<int>(v / p.token_bytes) < re,
+                      "V load of another head or past the range");
+            }
+        }
     }
 }
 
@@ -288,7 +299,7 @@ void window_loads(const Problem& pr, const PartialParams& p, const Buffers& buf,
 
 template <int D, int GT>
 void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage& cov, OutCoverage& out) {
-    constexpr int TPLV = kWave / (D / 4);  // FP32 kernel: token rows per 16-byte load group
+    constexpr int TPLV = kFp32TileTokens;
     const Buffers buf = buffers(pr);
     const Grid grid = partial_grid(p, pr.kv_heads);
     AUDIT(p.grid_x == grid.x && p.grid_y == grid.y, "kernel-argument grid %ux%u, launch %ux%u", p.grid_x, p.grid_y,
@@ -296,13 +307,8 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
     const int waves = partial_threads(p) / kWave;
     AUDIT(waves >= 1 && waves <= (p.row_mode ? kRowMaxWaves : 8), "workgroup of %d waves", waves);
     if (mfma) AUDIT(mfma_lds_bytes(p, D, pr.kv_elem) <= 160 * 1024, "LDS %d bytes", mfma_lds_bytes(p, D, pr.kv_elem));
-    const int align = mfma ? kTileTokens : kWave / (D / 4);
-    // Load groups per straight-line block and issued ahead, as the kernels'
-    // constants: matrix-core 2 and 2 (FP8 K/V outside whole rows: 4 and 4);
-    // FP32 16 and 4, whole-row FP32 launches 4 and 4.
-    const bool fp8_deep = mfma && pr.kv_elem == 1 && !p.row_mode;
-    const int block = mfma ? (fp8_deep ? 4 : 2) : p.row_mode ? 4 : 16;
-    const int ahead = mfma ? (fp8_deep ? 4 : 2) : 4, group_tokens = align;
+    const int align = mfma ? kTileTokens : kFp32TileTokens;
+    const int ring = mfma ? 2 : p.row_mode ? kFp32RowRing : kFp32Ring, group_tokens = align;  // tiles in flight per wave
     const int qw = p.quarters_per_wg;
     for (uint32_t bz = 0; bz < grid.z; ++bz) {
         for (uint32_t by = 0; by < grid.y; ++by) {
@@ -465,7 +471,7 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
                             g_own_passes += own.size();
                         }
                         // The kernels' token loop: page-id windows of 64 pages,
-                        // load groups issued `ahead` in blocks of `block`; a
+                        // `ring` tiles in flight and the next ring's requested; a
                         // shared-prefix item runs it once over the first
                         // member's row for the members that share it, then
                         // once per member with a row of its own.
@@ -478,18 +484,14 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
                                     window_loads(pr, p, buf, row_b, win);
                                 }
                                 re = imin(end, (win + kWave) << p.page_shift);
-                                for (int s0 = rb & ~(group_tokens - 1); s0 < re; s0 += block * group_tokens) {
+                                for (int s0 = rb & ~(group_tokens - 1); s0 < re; s0 += ring * group_tokens) {
                                     auto issue = [&](int t0) {
                                         if (mfma)
                                             mfma_tile<D>(pr, p, buf, w, row_b, t0, rb, re, win, wave, waves, len,
                                                          readers);
-                                        else fp32_group<D>(pr, p, buf, w, row_b, t0, rb, re, win, len);
+                                        else fp32_tile<D>(pr, p, buf, w, row_b, t0, rb, re, win, len);
                                     };
-                                    for (int n0 = 0; n0 < ahead; ++n0) issue(s0 + n0 * group_tokens);
-                                    for (int c = 0; c < block; ++c) {
-                                        if (s0 + c * group_tokens >= re) break;
-                                        if (c + ahead < block) issue(s0 + (c + ahead) * group_tokens);
-                                    }
+                                    for (int c = 0; c < 2 * ring; ++c) issue(s0 + c * group_tokens);
                                 }
                             }
                         };
