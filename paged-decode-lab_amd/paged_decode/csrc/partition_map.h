@@ -30,7 +30,6 @@ constexpr int kTileTokens = 16;  // tokens per matrix-core tile
 constexpr int kFp32TileTokens = 4;  // and per tile of the FP32 kernel: one MFMA's rows
 constexpr int kFp32Ring = 2;        // FP32 tiles in flight per wave
 constexpr int kFp32RowRing = 4;     // and of a whole-row wave, whose slice is few tiles
-constexpr int kMi355xCus = 256;  // compute units of an MI355X
 
 // Compacted work lists are passed in the kernel arguments for batches of up
 // to kCompactMaxBatch sequences. A tail item covers tail_span (at least
@@ -190,7 +189,7 @@ struct BlockCoords {
 
 template <int kList>
 PD_HD BlockCoords block_coords(uint32_t bx, uint32_t by, uint32_t bz, uint32_t gx, uint32_t gy, int xcd_shift,
-                               uint32_t xcd_main_rows, int xcd_tail_shift, int head_shift = -1) {
+                               uint32_t xcd_main_rows, int xcd_tail_shift, int head_shift) {
     if (xcd_shift >= 0) {
         const uint32_t x = bx & 7u;
         uint32_t r = by * 8u + x, tokens = bx >> 3;
@@ -1416,7 +1415,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
 
 // Launch shape of the FP32 kernel (and whole rows, as for the matrix-core
 // kernel).
-inline void plan_fp32(PartialParams& prm, int kv_heads, int head_dim, int cus = kMi355xCus) {
+inline void plan_fp32(PartialParams& prm, int kv_heads, int head_dim, int cus) {
     const int gt = head_tile(prm.group, 8);
     prm.head_tile = gt;
     prm.head_tiles = (prm.group + gt - 1) / gt;

@@ -49,6 +49,7 @@ struct Problem {
 uint64_t g_checks = 0;
 int g_failures = 0;
 bool g_plant_reach = false;  // --plant-reach: launch params that ignore the caller's partitions (negative control)
+bool g_plant_shift = false;  // --plant-shift: head groups one bit too wide in the grid's coordinates (negative control)
 bool g_plant_no_check = false;  // --plant-prefix: shared-prefix items that trust the runs (negative control)
 uint64_t g_own_passes = 0;      // shared-prefix members that read their own rows after the page check
 
@@ -107,7 +108,8 @@ PartialParams params(const Problem& pr, int cus, bool mfma, bool rows) {
     p.host_prefix_runs = pr.runs.empty() ? nullptr : pr.runs.data();
     plan_items(p, p.host_bounds);
     if (mfma) plan_mfma(p, pr.kv_heads, cus, pr.head_dim, pr.kv_elem);
-    else plan_fp32(p, pr.kv_heads, pr.head_dim);
+    else plan_fp32(p, pr.kv_heads, pr.head_dim, cus);
+    if (g_plant_shift && p.head_shift > 0) ++p.head_shift;
     return p;
 }
 
@@ -244,7 +246,11 @@ void mfma_tile(const Problem& pr, const PartialParams& p, const Buffers& buf, co
         const int n = lane % 16, g = lane / 16;
         for (int s = 0; s < KL; ++s) {
             const uint32_t off = tile_row_offset(p, TK * s + lane / KR, static_cast<uint32_t>(lane % KR) * 16u);
-            if (off < bytes) AUDIT(base + off + 16 <= buf.kv_bytes, "K load past the cache");
+            if (off < bytes) {
+                AUDIT(base + off + 16 <= buf.kv_bytes, "K load past the cache");
+                AUDIT(off % p.token_bytes + 16 <= D * ES + 0u && t0 + static_cast<int>(off / p.token_bytes) < re,
+                      "K load of another head or past the range");
+            }
             const int lds = wave * kTileTokens * stage_row + (TK * s + lane / KR) * stage_row + (lane % KR) * 16;
             AUDIT(lds >= 0 && lds + (ES == 2 ? 16 : 8) <= waves * mfma_stage_bytes(D, ES), "K stage write");
         }
@@ -254,7 +260,11 @@ void mfma_tile(const Problem& pr, const PartialParams& p, const Buffers& buf, co
         }
         for (int e = 0; e < 4; ++e) {
             const uint32_t off = tile_row_offset(p, 4 * e + g, static_cast<uint32_t>(n) * VH * ES);
-            if (off < bytes) AUDIT(base + off + 4u * VW <= buf.kv_bytes, "V load past the cache");
+            if (off < bytes) {
+                AUDIT(base + off + 4u * VW <= buf.kv_bytes, "V load past the cache");
+                AUDIT(off % p.token_bytes + 4u * VW <= D * ES + 0u && t0 + static_cast<int>(off / p.token_bytes) < re,
+                      "V load of another head or past the range");
+            }
         }
     }
 }
@@ -317,9 +327,9 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
                 const BlockCoords bc =
                     kind == kGridRectTails
                         ? block_coords<kGridRectTails>(bx, by, bz, p.grid_x, p.grid_y, p.xcd_shift, p.xcd_main_rows,
-                                                       p.xcd_tail_shift)
+                                                       p.xcd_tail_shift, p.head_shift)
                         : block_coords<kGridRect>(bx, by, bz, p.grid_x, p.grid_y, p.xcd_shift, p.xcd_main_rows,
-                                                  p.xcd_tail_shift);
+                                                  p.xcd_tail_shift, p.head_shift);
                 const int xcd = static_cast<int>((bx + static_cast<uint64_t>(grid.x) * (by + static_cast<uint64_t>(grid.y) * bz)) % 8);
                 const PartitionRange r = kind == kGridList        ? partition_range<kGridList>(p, bc)
                                          : kind == kGridRectTails ? partition_range<kGridRectTails>(p, bc)
@@ -357,7 +367,7 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
                 // caller's partitions; every read below is checked against it.
                 const int len = imax(0, imin(len_raw, reach_of(pr)));
                 const bool rows = p.row_mode != 0;
-                const int row_limit = mfma ? kRowMaxWaves : fp32_row_max_waves(GT);
+                const int row_limit = mfma ? row_max_waves(D) : fp32_row_max_waves(GT);
                 if (rows) {
                     AUDIT(!p.compact && waves == p.row_waves && waves <= row_limit, "whole-row launch of %d waves",
                           waves);
@@ -1449,6 +1459,17 @@ int main(int argc, char** argv) {
         std::vector<Problem> planted;
         for (const auto& pr : problems)
             if (pr.name.find(" prefix runs stale") != std::string::npos) planted.push_back(pr);
+        problems = planted;
+        appends.clear();
+        csrs.clear();
+    }
+    if (mode == "--plant-shift") {
+        // Negative control: plain grids whose coordinates take one bit too
+        // many for the head groups. The walk must report the states left out.
+        g_plant_shift = true;
+        std::vector<Problem> planted;
+        for (const auto& pr : problems)
+            if (pr.name.rfind("ragged shared B16 T32 split 128", 0) == 0) planted.push_back(pr);
         problems = planted;
         appends.clear();
         csrs.clear();

@@ -25,7 +25,7 @@ leave its buffer? -- is answered on the CPU:
   table conversion over valid and malformed metadata. Each kernel family has
   a planted-mistake negative control (wrong reach, merge live count, append
   capacity, missing CSR indices bound, shared-prefix items without their page
-  check) that the walk must report. It is
+  check, wrong head-group shift) that the walk must report. It is
   compiled with AddressSanitizer and UndefinedBehaviorSanitizer.
 * ``oracle/cpu_decode.c`` (the FP32 restatement the bench times) runs under
   the same sanitizers on ragged, empty-row, invalid-page-id and both-format
@@ -139,13 +139,15 @@ def test_partition_address_map_stays_in_bounds(audit_exe):
     ("--plant-append", "append reads table entry"),
     ("--plant-csr", "indices read 6 of 6"),
     ("--plant-prefix", "the item reads page"),
+    ("--plant-shift", "written 2 times, expected 1"),
 ])
 def test_address_audit_flags_planted_mistakes(audit_exe, plant, message):
     """Negative controls: launch parameters with one mistake planted (lengths
     clamped to the table instead of the caller's partitions; a merge live
     count one partition too long; an append capacity one page past the table;
     a CSR conversion without its bound on the indices read; shared-prefix
-    items that trust stale runs, without the kernel's page check). Each walk
+    items that trust stale runs, without the kernel's page check; grid
+    coordinates that shift by one bit too many). Each walk
     must report the accesses the mistake causes."""
     run = subprocess.run([str(audit_exe), plant], capture_output=True, text=True, timeout=300, env=ENV)
     assert run.returncode == 1, run.stdout[-4000:] + run.stderr[-4000:]
