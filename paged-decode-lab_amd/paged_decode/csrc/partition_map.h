@@ -973,11 +973,17 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
     const int64_t reach = lmin(static_cast<int64_t>(splits) * split_tokens, capacity);
     // Whether partitions of `span` tokens leave enough waves per CU:
     // kCoarseWavesPerCu, or kCoarseWavesRagged for lengths that are neither
-    // equal nor ragged enough for a work list. Shared-prefix items are not
-    // counted: measured with them, the ragged + shared B16 workload ran 27.2 us
-    // per staged call at the 512-token partitions this count picks and 32.5 us
-    // at 256 tokens, where counting the items' waves against 8 per CU would
-    // have stopped.
+    // equal nor ragged enough for a work list, in a call without shared-prefix
+    // items: those are formed by work lists, and one step coarser the partitions
+    // of such lengths are even enough for a rectangular grid, which reads the
+    // shared pages once per sequence. Measured on MI355X (decode call, us; 8
+    // against 6 waves, 25% of the pages shared): FP8 B18 L9434 ragged 39.5
+    // against 58.6, FP16 D 64 B6 L24344 42.1 against 51.1. The items' waves are
+    // not counted: the ragged + shared B16 workload ran 27.2 us per staged call
+    // at the 512-token partitions this count picks and 32.5 us at 256 tokens,
+    // where counting them against 8 per CU would have stopped.
+    const bool items = prefix_saving(prefix_runs, length_bounds, batch, reach, split_tokens, splits, page_shift,
+                                     slots).saved > 0;
     auto enough = [&](int64_t span) {
         int64_t parts = 0, most = 0, fewest = splits;
         for (int b = 0; b < batch; ++b) {
@@ -987,7 +993,7 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
             most = live > most ? live : most;
             fewest = lmin(fewest, live);
         }
-        const bool ragged = fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
+        const bool ragged = !items && fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
         return parts * kQuarters * kv_heads * head_tiles >=
                static_cast<int64_t>(ragged ? kCoarseWavesRagged : kCoarseWavesPerCu) * cus;
     };

@@ -636,6 +636,28 @@ def test_shared_prompt_samples_take_half_the_coarse_split(batch, context, shared
         assert grouped["kernel_split_tokens"] == 1024 and grouped["shared_prefix_items"] == 0
 
 
+@pytest.mark.parametrize("kv_dtype,batch,context,head_dim", [
+    (cabi.PD_DTYPE_FP8_E5M2, 18, 9434, 128),
+    (cabi.PD_DTYPE_F16, 12, 12000, 64),
+])
+def test_coarse_split_of_ragged_lengths_keeps_the_shared_prefix_items(kv_dtype, batch, context, head_dim):
+    """Ragged lengths (a quarter of the context to all of it) over a prompt that is a quarter of the pages: the full
+    call's split stops where its work list still scores the shared partitions for several sequences at once; without
+    sharing the same lengths run over coarser partitions."""
+    lib = cabi.load()
+    width = -(-context // 32)
+    table, pages = _sample_table(batch, width, width // 4)
+    runs = cabi.prefix_runs(lib, table)
+    lengths = np.linspace(context, context // 4, batch).astype(np.int32)
+    lengths[1:] = np.random.default_rng(batch).permutation(lengths[1:])
+    shape = (batch, 32, 8, head_dim, 32, width, pages, -(-context // 256), 256)
+    args = (cabi.PD_MERGE_SERIAL, cabi.PD_HINT_RAGGED_LENGTHS, lengths, 256)
+    grouped = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, kv_dtype, *shape, *args, runs)
+    plain = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, kv_dtype, *shape, *args)
+    assert grouped["shared_prefix_items"] > 0 and grouped["grid_kind"] == 2
+    assert plain["shared_prefix_items"] == 0 and plain["kernel_split_tokens"] >= 2 * grouped["kernel_split_tokens"]
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
