@@ -666,7 +666,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
     auto member_row = [&](int m) {
         return grouped ? static_cast<int64_t>(__shfl(member_b, m)) * p.query_heads + row_base : w.q_row;
     };
-    const int64_t col_row = member_row(col_member) + col_head;
+    // Formed again where it is used: kept, it would be spilled by the FP8 kernels
+    // of shared-prefix items. (All lanes together: it reads other lanes.)
+    auto col_row = [&] { return member_row(col_member) + col_head; };
     const int col_end = grouped ? min(max(__shfl(member_len, col_member), 0), p.reach) : 0x7FFFFFFF;
 
     // Page check of a shared-prefix item (prefix_span_pages): bit m of `own`
@@ -697,9 +699,10 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
     for (int s = 0; s < KS; ++s) {
         qb[s] = u32x4{0u, 0u, 0u, 0u};
         if (grouped) {
+            const int64_t row = col_row();
             if (col_live)
                 qb[s] = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.q) +
-                                                        (col_row * D + 32 * s + 8 * g) * 2);
+                                                        (row * D + 32 * s + 8 * g) * 2);
         } else if (n < w.heads_here) {
             qb[s] = *reinterpret_cast<const u32x4*>(q_row + (n * D + 32 * s + 8 * g) * 2);
         }
@@ -904,8 +907,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
         // Next member with a row of its own: its row, up to its own end.
         const int m = __builtin_ctz(pending);
         pending &= pending - 1;
-        pass_pages = p.table + static_cast<int64_t>(__builtin_amdgcn_readlane(member_b, m)) * p.table_width;
-        pass_end = min(w.we, min(max(__builtin_amdgcn_readlane(member_len, m), 0), p.reach));
+        const int b = __builtin_amdgcn_readlane(member_b, m);
+        pass_pages = p.table + static_cast<int64_t>(b) * p.table_width;
+        pass_end = min(w.we, min(max(p.lengths[b], 0), p.reach));
         col_on = col_member == m;
         window = -1;
     }
@@ -976,8 +980,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
             }
 #pragma unroll
             for (int j = 0; j < VH; ++j) slot->acc[j][lane] = acc[j];
+            const int64_t row = col_row();
             if (lane < 16 && col_live && part_first < col_end)
-                *reinterpret_cast<float2*>(p.stats + stats_offset(p, col_row, part)) = make_float2(kNoToken, 0.0f);
+                *reinterpret_cast<float2*>(p.stats + stats_offset(p, row, part)) = make_float2(kNoToken, 0.0f);
         }
         __syncthreads();
         if (qq != 0) return;
@@ -1016,8 +1021,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
                 dst[j / 4] = f32x4{acc[j][i], acc[j + 1][i], acc[j + 2][i], acc[j + 3][i]} * p.v_scale;
         }
     }
+    const int64_t row = col_row();
     if (lane < 16 && col_live && part_first < col_end) {
-        float2* st = reinterpret_cast<float2*>(p.stats + stats_offset(p, col_row, part));
+        float2* st = reinterpret_cast<float2*>(p.stats + stats_offset(p, row, part));
         *st = make_float2(l_head > 0.0f ? m_head : kNoToken, l_head);
     }
 }
