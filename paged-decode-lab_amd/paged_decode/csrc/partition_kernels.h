@@ -430,6 +430,14 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
 // ragged 39.5 -> 36.7; FP16 MQA B256 L2048 31.6 -> 28.2; B64 L8192 ragged 231 ->
 // 227. Two pairs in flight per wave (173 VGPRs and more, two waves per SIMD)
 // were slower: FP8 B4 15.3, FP16 B4 18.7, B16 ragged FP8 27.8 against 26.9.
+// Short ranges have nothing to overlap: a whole-row slice of one tile is read and
+// scored alone, with P.V over its 16 tokens, an empty second tile is not scored,
+// and a range's last pair requests nothing. Against pairs throughout (FP16, us):
+// 640 rows of up to 64 tokens with D 128 9.05 -> 7.36, 1088 rows of 32 7.66 ->
+// 6.08, MQA B256 of 256 tokens with D 64 10.14 -> 8.03, B16 of 640 tokens at split
+// 128 with twice the context reserved 16.6 -> 16.0; the copy of the computation
+// that this takes costs waves of two pairs up to 1.5% (64 / 8 heads B6 L4096 with
+// twice the context reserved 26.3 -> 26.7).
 //
 // FP8 K/V (OCP e4m3 or e5m2) are loaded as bytes and converted to the compute
 // type after they arrive; both formats convert exactly. The per-tensor scales
@@ -563,7 +571,7 @@ struct CombineSlot {
 // kFold: what the workgroup stores -- 0 one state per wave; 1 one state per
 // qw quarters of a partition (quarter combine); 2 the output rows of a whole
 // row's states (whole-row launch, up to kRowMaxWaves waves: 1024 lanes).
-template <typename QT, int KVF, int D, int GT, int NB, int kStream, int kFold, int kList>
+template <typename QT, int KVF, int D, int GT, int kStream, int kFold, int kList>
 __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave * 8, KVF == kKvNative ? 3 : 4)
     partial_mfma_kernel(const PartialParams p) {
     using C = Compute<QT>;
@@ -574,6 +582,7 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
     constexpr int VW = VH * ES / 4;               // stored words per V load
     static_assert(GT <= 16, "one MFMA column block holds at most 16 query heads");
     constexpr int kPair = 2;
+    constexpr bool kLastApart = last_pair_apart(kList, ES);
     constexpr int kPairTokens = kPair * kTileTokens;
 
     // K is loaded whole rows at a time (KR lanes x 16 bytes per token, TK
@@ -738,9 +747,11 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
         }
         return rq;
     };
-    auto load_k = [&](Pair& pr2, const Request& rq) {
+    // The next three take the tiles of a request that are used: kPair, or the
+    // first alone.
+    auto load_k = [&](auto tiles, Pair& pr2, const Request& rq) {
 #pragma unroll
-        for (int h = 0; h < kPair; ++h) {
+        for (int h = 0; h < decltype(tiles)::value; ++h) {
             const __amdgpu_buffer_rsrc_t kb = tile_buffer(k_head + rq.base[h], rq.bytes[h]);
 #pragma unroll
             for (int s = 0; s < KL; ++s)
@@ -748,9 +759,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto load_v = [&](Pair& pr2, const Request& rq) {
+    auto load_v = [&](auto tiles, Pair& pr2, const Request& rq) {
 #pragma unroll
-        for (int h = 0; h < kPair; ++h) {
+        for (int h = 0; h < decltype(tiles)::value; ++h) {
             const __amdgpu_buffer_rsrc_t vb = tile_buffer(v_head + rq.base[h], rq.bytes[h]);
 #pragma unroll
             for (int e = 0; e < VI; ++e)
@@ -793,11 +804,12 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
         return sc;
     };
 
-    // Softmax and P.V of the pair at t0, whose scores are sc.
-    auto accumulate = [&](Pair& pr2, const Request& rq, f32x4 (&sc)[kPair], int t0) {
+    // Softmax and P.V of the tiles at t0, whose scores are sc.
+    auto accumulate = [&](auto tiles, Pair& pr2, const Request& rq, f32x4 (&sc)[kPair], int t0) {
+        constexpr int NT = decltype(tiles)::value;
         float mx = -INFINITY;
 #pragma unroll
-        for (int h = 0; h < kPair; ++h) {
+        for (int h = 0; h < NT; ++h) {
             const int t1 = t0 + h * kTileTokens;
             // Whole tiles of an ungrouped item need no mask.
             if (grouped || rq.bytes[h] == 0u || t1 < rb || t1 + kTileTokens > re) {
@@ -828,9 +840,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
             }
         }
         // P in high and low parts, k = 8 g + 4 h + e <-> token g + 4 e of tile h.
-        u32x4 p_hi, p_lo;
+        u32x4 p_hi{}, p_lo{};
 #pragma unroll
-        for (int h = 0; h < kPair; ++h) {
+        for (int h = 0; h < NT; ++h) {
 #pragma unroll
             for (int e = 0; e < 4; e += 2) {
                 const float w0 = fast_exp2(fmaf(sc[h][e], p.scale_log2, -m_head));
@@ -847,9 +859,9 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
         constexpr int kWordDims = 4 / ES;
 #pragma unroll
         for (int w4 = 0; w4 < VW; ++w4) {
-            uint32_t vq[kPair][VI][kWordDims / 2];
+            uint32_t vq[NT][VI][kWordDims / 2];
 #pragma unroll
-            for (int h = 0; h < kPair; ++h)
+            for (int h = 0; h < NT; ++h)
 #pragma unroll
                 for (int e = 0; e < VI; ++e) {
                     const uint32_t raw[1] = {pr2.v[h][e][w4]};
@@ -857,50 +869,74 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
                 }
 #pragma unroll
             for (int j = 0; j < kWordDims; ++j) {
-                const u32x2 v0 = v_operand<kWordDims>(vq[0], j), v1 = v_operand<kWordDims>(vq[1], j);
-                const u32x4 vo = {v0[0], v0[1], v1[0], v1[1]};
+                const u32x2 v0 = v_operand<kWordDims>(vq[0], j);
                 f32x4& sum = acc[w4 * kWordDims + j];
-                sum = C::qk(p_hi, vo, sum);
-                sum = C::qk(p_lo, vo, sum);
+                if constexpr (NT == 1) {
+                    sum = C::pv(u32x2{p_hi[0], p_hi[1]}, v0, sum);
+                    sum = C::pv(u32x2{p_lo[0], p_lo[1]}, v0, sum);
+                } else {
+                    const u32x2 v1 = v_operand<kWordDims>(vq[1], j);
+                    const u32x4 vo = {v0[0], v0[1], v1[0], v1[1]};
+                    sum = C::qk(p_hi, vo, sum);
+                    sum = C::qk(p_lo, vo, sum);
+                }
             }
             if constexpr (KVF != kKvNative) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
+    constexpr std::integral_constant<int, 1> one{};
+    constexpr std::integral_constant<int, kPair> two{};
     uint32_t pending = own;
-    for (;;) {
+    if (kFold == 2 && one_tile_slice(w)) {
+        // A whole-row slice of one tile at most (short rows).
+        if (w.wb < w.we) {
+            if ((w.wb >> p.page_shift) != window) {
+                window = w.wb >> p.page_shift;
+                window_ids = pages[window_entry(p, window, lane)];
+            }
+            re = w.we;
+            Pair pair;
+            const Request at = locate(w.wb);
+            load_k(one, pair, at);
+            load_v(one, pair, at);
+            f32x4 sc[kPair];
+            sc[0] = score(pair, 0);
+            accumulate(one, pair, at, sc, w.wb);
+        }
+    } else for (;;) {
         for (rb = w.wb; rb < pass_end; rb = re) {
             if ((rb >> p.page_shift) != window) {
                 window = rb >> p.page_shift;
                 window_ids = pass_pages[window_entry(p, window, lane)];
             }
             re = min(pass_end, (window + kWave) << p.page_shift);
-            // A ring of NB pairs. Once a pair's K is scored, the K of the pair
-            // NB on is requested into its registers, and likewise V, so that
-            // loads are in flight while the wave computes. (Requests past the
-            // range are empty rather than skipped, and the loop has one exit:
-            // the compiler then counts the loads outstanding at every wait.)
-            Pair ring[NB];
-            Request at[NB];
-            int s0 = rb & ~(kTileTokens - 1);
+            // Once a pair's K is scored, the next pair's is requested into its
+            // registers, and likewise V, so that loads are in flight while the
+            // wave computes. The range's last pair, which requests nothing, is
+            // outside the loop (kLastApart): the compiler then counts the loads
+            // outstanding at every wait, as it could not past a request that is
+            // skipped.
+            int t0 = rb & ~(kTileTokens - 1);
+            Pair pair;
+            Request at = locate(t0);
+            load_k(two, pair, at);
+            load_v(two, pair, at);
+            f32x4 sc[kPair];
+            for (; t0 + (kLastApart ? kPairTokens : 0) < re; t0 += kPairTokens) {
 #pragma unroll
-            for (int c = 0; c < NB; ++c) {
-                at[c] = locate(s0 + c * kPairTokens);
-                load_k(ring[c], at[c]);
-                load_v(ring[c], at[c]);
+                for (int h = 0; h < kPair; ++h) sc[h] = score(pair, h);
+                const Request next = locate(t0 + kPairTokens);
+                load_k(two, pair, next);
+                accumulate(two, pair, at, sc, t0);
+                load_v(two, pair, next);
+                at = next;
             }
-            for (; s0 < re; s0 += NB * kPairTokens) {
-#pragma unroll
-                for (int c = 0; c < NB; ++c) {
-                    f32x4 sc[kPair];
-#pragma unroll
-                    for (int h = 0; h < kPair; ++h) sc[h] = score(ring[c], h);
-                    const Request next = locate(s0 + (NB + c) * kPairTokens);
-                    load_k(ring[c], next);
-                    accumulate(ring[c], at[c], sc, s0 + c * kPairTokens);
-                    load_v(ring[c], next);
-                    at[c] = next;
-                }
+            if constexpr (kLastApart) {
+                sc[0] = score(pair, 0);
+                sc[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (at.bytes[1] != 0u) sc[1] = score(pair, 1);
+                accumulate(two, pair, at, sc, t0);
             }
         }
         if (!grouped || pending == 0) break;
@@ -1030,9 +1066,6 @@ __global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave 
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? PD_OK : PD_ERR_LAUNCH; }
 
-// Matrix-core kernel: pairs of 16-token tiles in flight per wave.
-constexpr int kMfmaRing = 1;
-
 // Compute units of the current device, read once per device.
 inline int device_compute_units() {
     static std::atomic<int> cached[64];
@@ -1062,16 +1095,16 @@ int launch_mfma(const PartialParams& prm, int kv_heads, hipStream_t stream) {
 #define PD_LAUNCH_MFMA(MODE, FOLD)                                                                                \
     do {                                                                                                          \
         if constexpr (FOLD == 2)                                                                                  \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, 2, kGridRect>), \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, MODE, 2, kGridRect>), \
                                grid, block, lds, stream, prm);                                                    \
         else if (kind == kGridList)                                                                               \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, FOLD, kGridList>), grid,      \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, MODE, FOLD, kGridList>), grid,      \
                                block, lds, stream, prm);                                                          \
         else if (kind == kGridRectTails)                                                                          \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, FOLD, kGridRectTails>), grid, \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, MODE, FOLD, kGridRectTails>), grid, \
                                block, lds, stream, prm);                                                          \
         else                                                                                                      \
-            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, kMfmaRing, MODE, FOLD, kGridRect>), grid,      \
+            hipLaunchKernelGGL((partial_mfma_kernel<QT, KVF, D, GT, MODE, FOLD, kGridRect>), grid,      \
                                block, lds, stream, prm);                                                          \
     } while (0)
 #define PD_LAUNCH_MFMA_FOLDS(MODE)                      \

@@ -438,6 +438,17 @@ PD_HD WaveWork row_wave_work(const PartialParams& p, int b, int heads, int wave,
     return w;
 }
 
+// Whether a whole-row wave's slice is one tile of the matrix-core kernel at
+// most (slices start at tiles).
+PD_HD bool one_tile_slice(const WaveWork& w) { return w.we - w.wb <= kTileTokens; }
+
+// Whether the matrix-core kernel of a grid kind computes a range's last pair of
+// tiles apart from its loop, which then requests nothing past the range. A
+// second copy of a pair's computation does not fit the registers of the FP8
+// kernels whose items may be shared-prefix ones (2 to 4 spilled): their requests
+// past a range are empty instead.
+constexpr bool last_pair_apart(int kind, int elem) { return kind != kGridList || elem == 2; }
+
 // First logical page of a whole-row wave's slice if the row is full length.
 template <int ALIGN>
 PD_HD int row_speculative_page(const PartialParams& p, int wave, int waves) {

@@ -8,8 +8,9 @@
 // partition_range, wave_work, speculative_page, window_entry, tile_slot,
 // tile_live, tile_base, tile_bytes, tile_row_offset, numerator_offset,
 // stats_offset), following the kernels' loop structure (page-id windows of 64
-// entries, a ring of two 16-token tiles for the matrix-core kernel and of
-// kFp32Ring or kFp32RowRing 4-token ones for the FP32 kernel, each requested again one ring on).
+// entries, pairs of 16-token tiles for the matrix-core kernel, the next pair
+// requested while one is computed, or the one tile of a short whole-row slice,
+// and rings of kFp32Ring or kFp32RowRing 4-token tiles for the FP32 kernel).
 // Every global load that its buffer descriptor lets through is
 // checked to lie inside q, k, v, table or lengths, every store inside numerator or stats, every LDS access
 // inside the launch's dynamic LDS; every live token is read from the page its
@@ -319,6 +320,7 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
     if (mfma) AUDIT(mfma_lds_bytes(p, D, pr.kv_elem) <= 160 * 1024, "LDS %d bytes", mfma_lds_bytes(p, D, pr.kv_elem));
     const int align = mfma ? kTileTokens : kFp32TileTokens;
     const int ring = mfma ? 2 : p.row_mode ? kFp32RowRing : kFp32Ring, group_tokens = align;  // tiles in flight per wave
+    const bool last_apart = mfma && last_pair_apart(grid_kind(p), pr.kv_elem);
     const int qw = p.quarters_per_wg;
     for (uint32_t bz = 0; bz < grid.z; ++bz) {
         for (uint32_t by = 0; by < grid.y; ++by) {
@@ -494,14 +496,25 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
                                     window_loads(pr, p, buf, row_b, win);
                                 }
                                 re = imin(end, (win + kWave) << p.page_shift);
-                                for (int s0 = rb & ~(group_tokens - 1); s0 < re; s0 += ring * group_tokens) {
-                                    auto issue = [&](int t0) {
+                                int s0 = rb & ~(group_tokens - 1);
+                                auto request = [&](int t0, int tiles) {
+                                    for (int c = 0; c < tiles; ++c) {
+                                        const int t = t0 + c * group_tokens;
                                         if (mfma)
-                                            mfma_tile<D>(pr, p, buf, w, row_b, t0, rb, re, win, wave, waves, len,
+                                            mfma_tile<D>(pr, p, buf, w, row_b, t, rb, re, win, wave, waves, len,
                                                          readers);
-                                        else fp32_tile<D>(pr, p, buf, w, row_b, t0, rb, re, win, len);
-                                    };
-                                    for (int c = 0; c < 2 * ring; ++c) issue(s0 + c * group_tokens);
+                                        else fp32_tile<D>(pr, p, buf, w, row_b, t, rb, re, win, len);
+                                    }
+                                };
+                                if (mfma && rows && one_tile_slice(w)) {
+                                    AUDIT(s0 == w.wb && re == w.we, "slice [%d, %d) is not one tile", w.wb, w.we);
+                                    request(s0, 1);
+                                    continue;
+                                }
+                                request(s0, ring);
+                                for (; s0 + (last_apart ? ring * group_tokens : 0) < re; s0 += ring * group_tokens) {
+                                    if (last_apart) AUDIT(s0 + ring * group_tokens < re, "request past the range");
+                                    request(s0 + ring * group_tokens, ring);
                                 }
                             }
                         };

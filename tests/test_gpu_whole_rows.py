@@ -172,6 +172,34 @@ def test_whole_rows_graph_replay(q_dtype):
         assert torch.equal(plan._out, eager)
 
 
+@pytest.mark.parametrize("q_dtype,kv_dtype", FORMATS)
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [(8, 8, 128, 16), (20, 4, 64, 32), (16, 1, 128, 16), (35, 5, 64, 16)])
+@pytest.mark.parametrize("tokens", [16, 48, 128])
+def test_short_slices_match_oracle(q_dtype, kv_dtype, heads, kv_heads, dim, page, tokens):
+    """Slices of no, one and two tiles in one workgroup: every row length around the tiles' edges, private pages. Slots
+    that hold no live token are NaN, so a tile read or summed past a slice's end would show."""
+    announce(f"short slices q={q_dtype} kv={kv_dtype} {heads}/{kv_heads} D{dim} T{page} up to {tokens}")
+    edges = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 63, 65, 100, 127, 128]
+    lengths = np.array([tokens] + [n for n in edges if n <= tokens], dtype=np.int32)
+    width = -(-tokens // page)
+    layout = Layout(len(lengths), heads, kv_heads, dim, page, len(lengths) * width)
+    table = np.random.default_rng(tokens).permutation(layout.physical_pages).reshape(-1, width).astype(np.int32)
+    (q, k, v), (k_scale, v_scale), exact = device_inputs(layout, q_dtype, kv_dtype, seed=heads)
+    dead = torch.ones((layout.physical_pages, page), dtype=torch.bool)
+    for b, n in enumerate(lengths):
+        pos = np.arange(n)
+        dead[table[b, pos // page], pos % page] = False
+    for t in (k, v):
+        poisoned = t.float()
+        poisoned[dead.to(t.device)] = float("nan")
+        t.copy_(poisoned.to(t.dtype))
+    plan = DecodePlan(layout, table, lengths, split_tokens=128)
+    assert plan.launches(q.dtype, k.dtype) == 1
+    out = plan.run(q, k, v, k_scale=k_scale, v_scale=v_scale).cpu().numpy()
+    assert_parity(out, dense_attention(*exact, table, lengths), bar(q_dtype))
+    np.testing.assert_array_equal(out[lengths == 0], 0.0)
+
+
 # (batch, query heads, KV heads, head_dim, tokens per row, launches on 256 CUs): rows on each side of the launch's
 # bounds (7/8 of the CUs for 256 KB, one per CU for 512 KB) and of its workgroup sizes (8 or 16 waves, 4, 2, 1).
 LARGE = [
