@@ -571,8 +571,15 @@ struct CombineSlot {
 // kFold: what the workgroup stores -- 0 one state per wave; 1 one state per
 // qw quarters of a partition (quarter combine); 2 the output rows of a whole
 // row's states (whole-row launch, up to kRowMaxWaves waves: 1024 lanes).
+//
+// The waves per SIMD are those that the registers allow without a spill: left to
+// itself the compiler takes 5 to 16 more for D 64 (FP16, 5 KV heads B32 L3000 with
+// twice the context reserved: 22.6 -> 20.8 us).
+constexpr int mfma_waves_per_simd(int head_dim, int elem) { return head_dim == 64 ? 5 : elem == 2 ? 3 : 4; }
+
 template <typename QT, int KVF, int D, int GT, int kStream, int kFold, int kList>
-__global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave * 8, KVF == kKvNative ? 3 : 4)
+__global__ void __launch_bounds__(kFold == 2 ? kWave * row_max_waves(D) : kWave * 8,
+                                  mfma_waves_per_simd(D, KVF == kKvNative ? 2 : 1))
     partial_mfma_kernel(const PartialParams p) {
     using C = Compute<QT>;
     constexpr int ES = KVF == kKvNative ? 2 : 1;  // stored bytes per K/V element
