@@ -970,6 +970,7 @@ inline int prefix_finer_split(int c, const int32_t* runs, const int32_t* bounds,
 // prefix_finer_split may halve c.
 constexpr int64_t kCoarseWaveBytes = 128 * 1024;
 constexpr int kCoarseWavesRagged = 6;
+constexpr int kItemSplitTokens = 1024;
 
 struct KernelSplit {
     int splits, split_tokens;
@@ -984,13 +985,15 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
     const int64_t reach = lmin(static_cast<int64_t>(splits) * split_tokens, capacity);
     // Whether partitions of `span` tokens leave enough waves per CU:
     // kCoarseWavesPerCu, or kCoarseWavesRagged for lengths that are neither
-    // equal nor ragged enough for a work list, in a call without shared-prefix
-    // items: those are formed by work lists, and one step coarser the partitions
-    // of such lengths are even enough for a rectangular grid, which reads the
-    // shared pages once per sequence. Measured on MI355X (decode call, us; 8
-    // against 6 waves, 25% of the pages shared): FP8 B18 L9434 ragged 39.5
-    // against 58.6, FP16 D 64 B6 L24344 42.1 against 51.1. The items' waves are
-    // not counted: the ragged + shared B16 workload ran 27.2 us per staged call
+    // equal nor ragged enough for a work list, unless shared-prefix items are
+    // lost by it: those are formed by work lists, and one step coarser the
+    // partitions of such lengths are even enough for a rectangular grid, which
+    // reads the shared pages once per sequence. Measured on MI355X (decode call,
+    // us; 8 against 6 waves, a quarter of the pages shared): from 1024 to 2048
+    // tokens FP8 B18 L9434 ragged 44.0 against 58.7, FP16 D 64 B6 L24344 42.6
+    // against 52.5; but up to kItemSplitTokens longer partitions are worth more:
+    // 16 KV heads B16 L2048, 512 to 1024 tokens, FP8 24.4 against 19.6, FP16 D 64
+    // 20.6 against 17.1. The items' waves are not counted: the ragged + shared B16 workload ran 27.2 us per staged call
     // at the 512-token partitions this count picks and 32.5 us at 256 tokens,
     // where counting them against 8 per CU would have stopped.
     const bool items = prefix_saving(prefix_runs, length_bounds, batch, reach, split_tokens, splits, page_shift,
@@ -1004,7 +1007,7 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
             most = live > most ? live : most;
             fewest = lmin(fewest, live);
         }
-        const bool ragged = !items && fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
+        const bool ragged = (!items || span <= kItemSplitTokens) && fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
         return parts * kQuarters * kv_heads * head_tiles >=
                static_cast<int64_t>(ragged ? kCoarseWavesRagged : kCoarseWavesPerCu) * cus;
     };

@@ -658,6 +658,19 @@ def test_coarse_split_of_ragged_lengths_keeps_the_shared_prefix_items(kv_dtype, 
     assert plain["shared_prefix_items"] == 0 and plain["kernel_split_tokens"] >= 2 * grouped["kernel_split_tokens"]
 
 
+def test_coarse_split_of_short_shared_contexts_prefers_longer_partitions():
+    """16 KV heads, ragged contexts of up to 2048 tokens, a quarter shared: 1024-token partitions, whose longer quarters
+    are worth more than shared-prefix items over 512."""
+    lib = cabi.load()
+    table, pages = _sample_table(16, 64, 16)
+    lengths = np.linspace(2048, 512, 16).astype(np.int32)
+    lengths[1:] = np.random.default_rng(16).permutation(lengths[1:])
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_FP8_E4M3, 16, 64, 16, 128, 32, 64, pages, 8, 256,
+                            cabi.PD_MERGE_SERIAL, cabi.PD_HINT_RAGGED_LENGTHS, lengths, 256,
+                            cabi.prefix_runs(lib, table))
+    assert plan["kernel_split_tokens"] == 1024
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
