@@ -663,8 +663,8 @@ def test_coarse_split_of_short_shared_contexts_prefers_longer_partitions():
     are worth more than shared-prefix items over 512."""
     lib = cabi.load()
     table, pages = _sample_table(16, 64, 16)
-    lengths = np.linspace(2048, 512, 16).astype(np.int32)
-    lengths[1:] = np.random.default_rng(16).permutation(lengths[1:])
+    lengths = np.random.default_rng(1).integers(512, 2049, 16).astype(np.int32)
+    lengths[0] = 2048
     plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_FP8_E4M3, 16, 64, 16, 128, 32, 64, pages, 8, 256,
                             cabi.PD_MERGE_SERIAL, cabi.PD_HINT_RAGGED_LENGTHS, lengths, 256,
                             cabi.prefix_runs(lib, table))
