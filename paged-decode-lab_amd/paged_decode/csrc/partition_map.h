@@ -1285,6 +1285,36 @@ PD_HD MergeRow merge_xcd_row(uint32_t bx, uint32_t by, int group_rows, int xcd_s
                     static_cast<int64_t>(r) * group_rows + static_cast<int64_t>(bx >> 3) * unit + sub};
 }
 
+// Whether workgroups of 8 or 6 waves (4 or 3 KV heads x 2 quarters) are better
+// halved -- 4 or 8 KV heads to 2 heads x 2 quarters, others to one quarter of
+// their heads: on a rectangular grid when the most loaded CU then holds fewer
+// waves (12 instead of 16 at 12 waves per CU; tail items are not counted; grids of
+// more than 16 are dealt out as CUs get free; up to 4 is a small grid), on a work list, whose items differ, while they leave it at most kHalvedListWaves
+// waves per CU. Measured on MI355X (decode call, us, 8 -> 4 waves): at 12 waves per CU FP8 B6 L4096 16.2 ->
+// 15.5, B24 L2048 ragged 21.4 -> 19.4, B12 L8192 ragged 37.5 -> 32.7, FP16 D 64 B6
+// 15.0 -> 14.0, B12 L8192 ragged 34.8 -> 30.4, 4 KV heads B24 L2048 13.9 -> 12.7;
+// at 6, 8 or 16 FP8 B6 L4096 with 4 KV heads 10.2 -> 10.7, B32 L4096 ragged 35.8 ->
+// 37.0, D 64 with twice the context reserved 25.6 -> 27.4, FP16 D 64 B32 L4096
+// empty to full 30.3 -> 32.6; work lists at 10 to 13 FP8 B32 L4096 half shared
+// 42.6 -> 33.7, a quarter shared 26.2 -> 22.9, FP16 D 64 22.6 -> 20.0, at 15 to 17
+// FP8 D 64 B12 L8192 half shared 20.8 -> 22.9, B64 L2048 14.0 -> 14.4. With 16 KV
+// heads, 4 x 2 -> 4 x 1 (2 x 2): FP8 B6 L4096 ragged 21.0 -> 17.7 (19.3), D 64 with
+// twice the context reserved 19.3 -> 15.4 (18.8), FP16 D 64 22.6 -> 18.8 (20.5);
+// with 3, 3 x 2 -> 3 x 1: FP16 D 64 B32 L3000 ragged 18.6 -> 15.8.
+constexpr int kHalvedListWaves = 14;
+
+inline bool prefers_half_workgroups(const PartialParams& prm, int kv_heads, int cus) {
+    if (prm.compact) {
+        const PrefixSaving s = prefix_saving(prm.host_prefix_runs, prm.host_bounds, prm.batch, prm.reach,
+                                             prm.split_tokens, prm.splits, prm.page_shift, prefix_slots(prm.group));
+        return item_workgroups(prm, kv_heads, prm.items - s.saved) * (partial_threads(prm) / kWave) <=
+               static_cast<int64_t>(kHalvedListWaves) * cus;
+    }
+    const int64_t whole = shape_workgroups(prm, kv_heads), waves = whole * (partial_threads(prm) / kWave);
+    if (waves <= 4ll * cus || waves > 16ll * cus) return false;
+    return (2 * whole + cus - 1) / cus < 2 * ((whole + cus - 1) / cus);
+}
+
 // Launch shape of the matrix-core kernel on a device of `cus` compute units,
 // for head_dim and K/V elements of elem bytes: head tile, workgroup shape,
 // quarter combine or whole rows, and streaming mode.
@@ -1312,6 +1342,10 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     // heads 25.1 and 26.1.
     const bool wide = head_dim * elem >= 256;
     choose_workgroup(prm, kv_heads, wide ? 2 : 4, !wide && kv_heads > 2 ? 8 : prm.head_tiles > 1 ? 6 : 4);
+    const int whole_heads = prm.heads_per_wg;
+    const bool halved = partial_threads(prm) > 4 * kWave && prm.quarters_per_wg == 2 && gt <= 8 &&
+                        prefers_half_workgroups(prm, kv_heads, cus);
+    if (halved) choose_workgroup(prm, kv_heads, kv_heads == 4 || kv_heads == 8 ? 2 : 4, 4);
     if (prm.heads_per_wg == 1 && kv_heads > 1 && kv_heads <= 8 && prm.head_tiles == 1) {
         prm.heads_per_wg = kv_heads;
         prm.quarters_per_wg = 1;
@@ -1364,7 +1398,12 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     prm.combine = fills_device && (prm.quarters_per_wg == 2 || (prm.quarters_per_wg == 4 && gt == 16));
     const bool long_quarters = fills_device && waves_total > 4ll * cus && gt <= 8 && kv_heads <= 8 && elem == 2 &&
                                !prm.ragged_lengths && prm.split_tokens >= 1024;
-    const int default_groups = kv_heads / prm.heads_per_wg;
+    // Halved workgroups count the head groups of whole ones, but work lists of
+    // slices of whole cache lines the halved ones (FP8, shared pages, by whole /
+    // halved groups: D 128 lists B32 L4096 half shared 39.3 / 33.7, D 64 22.5 / 25.5;
+    // rectangular D 128 B6 L4096 12.3 / 12.8).
+    const bool count_whole = halved && !(prm.compact && head_dim * elem >= 128);
+    const int default_groups = kv_heads / (count_whole ? whole_heads : prm.heads_per_wg);
     // When the KV heads need several workgroups (kv_heads > heads_per_wg),
     // each workgroup reads one head group's slice of every token row, and
     // some 16-byte loads may be issued non-temporal. That is faster when

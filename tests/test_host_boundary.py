@@ -671,6 +671,37 @@ def test_coarse_split_of_short_shared_contexts_prefers_longer_partitions():
     assert plan["kernel_split_tokens"] == 1024
 
 
+@pytest.mark.parametrize("kv_dtype,heads,kv_heads,dim,batch,context,expected", [
+    (cabi.PD_DTYPE_FP8_E4M3, 32, 8, 128, 6, 4096, (4, 2)),    # 12 waves per CU: 3 workgroups of 4 on each, not 2 or 1 of 8
+    (cabi.PD_DTYPE_F16, 32, 8, 64, 24, 2048, (4, 2)),
+    (cabi.PD_DTYPE_FP8_E4M3, 64, 16, 64, 6, 4096, (4, 4)),    # more heads: one quarter of four
+    (cabi.PD_DTYPE_FP8_E4M3, 12, 3, 128, 32, 3072, (3, 3)),   # 9 per CU: 3 x 3 waves, not 2 or 1 of 6
+    (cabi.PD_DTYPE_FP8_E4M3, 32, 8, 128, 32, 4096, (8, 4)),   # whole rounds: 8 per CU
+    (cabi.PD_DTYPE_FP8_E4M3, 16, 4, 128, 6, 4096, (8, 4)),    # 6 per CU: 8 on the most loaded CU either way
+    (cabi.PD_DTYPE_FP8_E4M3, 32, 8, 64, 146, 4096, (8, 4)),   # more than 16 per CU: dealt out as CUs get free
+])
+def test_workgroups_of_small_head_slices_load_the_cus_evenly(kv_dtype, heads, kv_heads, dim, batch, context, expected):
+    """Waves and KV heads per workgroup of equal-length calls over 128-byte slices or less (split 256, 256 CUs)."""
+    lib = cabi.load()
+    width = 2 * context // 16  # twice the context reserved: tail items do not count
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, kv_dtype, batch, heads, kv_heads, dim, 16, width, batch * width,
+                            width // 16, 256, cabi.PD_MERGE_SERIAL, cabi.PD_HINT_UNSHARED_PAGES,
+                            np.full(batch, context, dtype=np.int32), 256)
+    assert (plan["waves_per_workgroup"], plan["kv_heads_per_workgroup"]) == expected
+
+
+@pytest.mark.parametrize("batch,context,waves", [(32, 4096, 4), (24, 2048, 8)])
+def test_work_lists_of_small_head_slices_take_small_workgroups(batch, context, waves):
+    """FP8 lists of samples of one prompt, half of it shared (10 and 15 waves per CU)."""
+    lib = cabi.load()
+    width = context // 32
+    table, pages = _sample_table(batch, width, width // 2)
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_FP8_E4M3, batch, 32, 8, 128, 32, width, pages,
+                            context // 256, 256, cabi.PD_MERGE_SERIAL, cabi.PD_HINT_NONE,
+                            np.full(batch, context, dtype=np.int32), 256, cabi.prefix_runs(lib, table))
+    assert plan["shared_prefix_items"] > 0 and plan["waves_per_workgroup"] == waves
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
