@@ -761,6 +761,15 @@ inline int mfma_lds_bytes(const PartialParams& prm, int head_dim, int elem) {
 //   - kRowMaxBytesFull: when the rows come to at least kRowFill of the CUs.
 //   - kRowMaxBytesRound: when, besides, they are at most one per CU, so that
 //     no CU waits for others' second row.
+//   - kRowMaxBytesPart when, besides, a head's slice of a token row is part of a
+//     cache line (FP8, D 64): the workgroups of neighbouring heads, on other
+//     XCDs, then read the same lines. FP8 D 64 with 8 KV heads, rows against two
+//     launches: 256 KB, 256 rows 24.6 against 17.5, 512 rows ragged 32.3 against
+//     24.8, 512 KB 44.4 against 28.3; 160 KB, 256 rows 16.9 against 15.8, ragged
+//     512 rows 22.1 against 24.9; one KV head (whole lines) 512 KB 26.0 against 27.5.
+//     Not without host bounds, where two launches keep the caller's split and
+//     its dead partitions: 512 rows of up to 1000 tokens, 2000 reserved, 20.8
+//     against 28.7.
 // Calls that may form shared-prefix items (shared_prefixes) keep the first
 // bound: their partition launch reads a shared page once for several rows.
 // Measured on MI355X (decode call, us, graph; GQA 4, D 128, FP16; two launches
@@ -774,15 +783,19 @@ inline int mfma_lds_bytes(const PartialParams& prm, int head_dim, int elem) {
 constexpr int64_t kRowMaxBytes = 128 * 1024;
 constexpr int64_t kRowMaxBytesFull = 256 * 1024;
 constexpr int64_t kRowMaxBytesRound = 512 * 1024;
+constexpr int64_t kRowMaxBytesPart = 160 * 1024;
+constexpr int kCacheLine = 128;
 constexpr int kRowFill = 7;  // eighths of the CUs
 constexpr int kRowWaveTokens = 16;
 
 // Whether a call's rows -- `rows` of `reach` tokens (PartialParams::reach) of K
 // and V each, elem bytes per element -- are small enough for a whole-row launch.
-inline bool rows_fit_one_launch(int64_t rows, int64_t reach, int head_dim, int elem, int cus, bool shared_prefixes) {
+inline bool rows_fit_one_launch(int64_t rows, int64_t reach, int kv_heads, int head_dim, int elem, int cus,
+                                bool bounded, bool shared_prefixes) {
     const int64_t bytes = reach * head_dim * elem * 2;
     if (bytes <= kRowMaxBytes) return true;
     if (shared_prefixes || rows * 8 < static_cast<int64_t>(cus) * kRowFill) return false;
+    if (bounded && kv_heads > 1 && head_dim * elem < kCacheLine && bytes > kRowMaxBytesPart) return false;
     return bytes <= kRowMaxBytesFull || (bytes <= kRowMaxBytesRound && rows <= cus);
 }
 
@@ -1089,7 +1102,7 @@ inline void plan_rows(PartialParams& prm, int kv_heads, int head_dim, int elem, 
     prm.row_mode = 0;
     if (!prm.row_allowed) return;
     const int64_t rows = static_cast<int64_t>(prm.batch) * kv_heads * prm.head_tiles;
-    if (!rows_fit_one_launch(rows, prm.reach, head_dim, elem, cus,
+    if (!rows_fit_one_launch(rows, prm.reach, kv_heads, head_dim, elem, cus, prm.host_bounds != nullptr,
                              may_share_prefixes(prm.host_prefix_runs, prm.host_bounds, prm.batch, slots)))
         return;
     const int64_t span = prm.reach;
@@ -1402,7 +1415,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     // slices of whole cache lines the halved ones (FP8, shared pages, by whole /
     // halved groups: D 128 lists B32 L4096 half shared 39.3 / 33.7, D 64 22.5 / 25.5;
     // rectangular D 128 B6 L4096 12.3 / 12.8).
-    const bool count_whole = halved && !(prm.compact && head_dim * elem >= 128);
+    const bool count_whole = halved && !(prm.compact && head_dim * elem >= kCacheLine);
     const int default_groups = kv_heads / (count_whole ? whole_heads : prm.heads_per_wg);
     // When the KV heads need several workgroups (kv_heads > heads_per_wg),
     // each workgroup reads one head group's slice of every token row, and

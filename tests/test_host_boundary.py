@@ -702,6 +702,22 @@ def test_work_lists_of_small_head_slices_take_small_workgroups(batch, context, w
     assert plan["shared_prefix_items"] > 0 and plan["waves_per_workgroup"] == waves
 
 
+@pytest.mark.parametrize("kv_heads,dim,batch,tokens,bounded,launches", [
+    (8, 64, 64, 2048, True, 2),    # 64 bytes of each line: two launches
+    (8, 64, 64, 1280, True, 1),    # 160 KB rows
+    (1, 64, 256, 2048, True, 1),   # one KV head: whole lines
+    (8, 128, 32, 1024, True, 1),   # 128-byte slices
+    (8, 64, 64, 2048, False, 1),   # lengths known on the device only
+])
+def test_large_rows_of_partial_cache_lines_take_two_launches(kv_heads, dim, batch, tokens, bounded, launches):
+    lib = cabi.load()
+    width = tokens // 16
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_FP8_E4M3, batch, 4 * kv_heads, kv_heads, dim, 16,
+                            width, batch * width, tokens // 256, 256, cabi.PD_MERGE_SERIAL,
+                            cabi.PD_HINT_UNSHARED_PAGES, np.full(batch, tokens, dtype=np.int32) if bounded else None, 256)
+    assert plan["launches"] == launches
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
