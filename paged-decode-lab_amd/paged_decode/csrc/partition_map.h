@@ -1069,7 +1069,10 @@ constexpr int fp32_row_max_waves(int gt) { return gt >= 8 ? 8 : kRowMaxWaves; }
 // CU can cover, and each wave brings 4 to 13 KB of LDS:
 //   - Rows that fit the CUs at once take 8 waves, or one lane per output
 //     element where that is more (a fold in one pass): 16-wave workgroups cost
-//     more to start and to fold than their shorter slices save.
+//     more to start and to fold than their shorter slices save. Larger rows
+//     whose fold takes several passes with any workgroup keep 8 (16 heads of 128
+//     dims, 256 rows of 512 tokens FP16 19.6 with 12 waves, 18.4 with 8; ragged
+//     16.9 and 15.5; 1024 tokens ragged 23.8 and 22.7).
 //   - From one row per CU on, 4 waves, so that several workgroups share a CU.
 //   - From four rows per CU on, waves of at least kRowWaveBytes each, but two
 //     of them up to eight rows per CU: the other rows fill the CU.
@@ -1087,7 +1090,11 @@ constexpr int kRowWavesFew = 8;
 constexpr int kRowWavesMany = 4;
 
 inline int row_waves_for(int64_t rows, int64_t row_bytes, int outputs, int max_waves, int cus) {
-    if (rows <= cus) return imin(max_waves, imax(kRowWavesFew, (outputs + kWave - 1) / kWave));
+    if (rows <= cus) {
+        const int one_pass = (outputs + kWave - 1) / kWave;
+        if (row_bytes > kRowMaxBytes && one_pass > max_waves) return imin(max_waves, kRowWavesFew);
+        return imin(max_waves, imax(kRowWavesFew, one_pass));
+    }
     int waves = imin(max_waves, kRowWavesMany);
     if (rows >= 4ll * cus)
         waves = static_cast<int>(lmin(waves, imax(rows >= 8ll * cus ? 1 : 2, static_cast<int>(row_bytes / kRowWaveBytes))));

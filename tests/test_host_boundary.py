@@ -718,6 +718,20 @@ def test_large_rows_of_partial_cache_lines_take_two_launches(kv_heads, dim, batc
     assert plan["launches"] == launches
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,batch,tokens,waves", [
+    (64, 8, 128, 28, 512, 8), (16, 1, 128, 256, 512, 8),   # 1024 and 2048 outputs: several passes over 12 waves too
+    (32, 8, 128, 28, 512, 8), (16, 1, 64, 256, 1024, 16),  # one pass over 8 and over 16 waves
+    (64, 8, 128, 28, 192, 12),                             # short rows keep one wave per tile
+])
+def test_waves_of_large_rows(heads, kv_heads, dim, batch, tokens, waves):
+    lib = cabi.load()
+    width = tokens // 16
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_F16, batch, heads, kv_heads, dim, 16, width,
+                            batch * width, -(-tokens // 256), 256, cabi.PD_MERGE_SERIAL, cabi.PD_HINT_UNSHARED_PAGES,
+                            np.full(batch, tokens, dtype=np.int32), 256)
+    assert plan["launches"] == 1 and plan["waves_per_workgroup"] == waves
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
