@@ -1335,6 +1335,26 @@ inline bool prefers_half_workgroups(const PartialParams& prm, int kv_heads, int 
     return (2 * whole + cus - 1) / cus < 2 * ((whole + cus - 1) / cus);
 }
 
+// Whether the 4-wave workgroups (2 KV heads x 2 quarters) of 256-byte head slices
+// are better doubled to 4 heads, 1 KB of each token row: from 16 KV heads and
+// kWideTokens-token partitions on, on a rectangular grid whose live workgroups
+// fill at least 3/4 of their rounds over the CUs, an eighth of a round more not
+// counted (such a workgroup holds a CU alone). Measured on MI355X (decode call, us, 2 -> 4 heads, FP16): 32 KV heads
+// B2 L11032 ragged with a quarter of the pages shared 45.4 -> 39.8, B16 L2048
+// ragged 65.9 -> 60.5, B4 L4096 ragged 32.9 -> 30.9, B8 88.9 -> 86.8; 16 KV heads B16 L2048 45.9 -> 43.9;
+// rounds filled to 0.7 32 KV heads B2 L11032 61.3 -> 65.4, B8 L4096 ragged 57.7 -> 60.7;
+// 512-token partitions 16 KV heads B8 L4096 ragged 30.6 -> 33.4; work lists B8
+// L4096 half shared 61.3 -> 68.5.
+constexpr int kWideTokens = 1024;
+
+inline bool prefers_wide_workgroups(const PartialParams& prm, int kv_heads, int cus) {
+    if (kv_heads < 16 || kv_heads % 4 != 0 || prm.head_tiles > 1 || prm.compact || prm.split_tokens < kWideTokens)
+        return false;
+    const int64_t live = static_cast<int64_t>(prm.live_items) * 2 * (kv_heads / 4);
+    const int64_t rounds = (live + cus - 1 - cus / 8) / cus;
+    return rounds > 0 && live * 4 >= rounds * cus * 3;
+}
+
 // Launch shape of the matrix-core kernel on a device of `cus` compute units,
 // for head_dim and K/V elements of elem bytes: head tile, workgroup shape,
 // quarter combine or whole rows, and streaming mode.
@@ -1366,6 +1386,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     const bool halved = partial_threads(prm) > 4 * kWave && prm.quarters_per_wg == 2 && gt <= 8 &&
                         prefers_half_workgroups(prm, kv_heads, cus);
     if (halved) choose_workgroup(prm, kv_heads, kv_heads == 4 || kv_heads == 8 ? 2 : 4, 4);
+    if (wide && prefers_wide_workgroups(prm, kv_heads, cus)) choose_workgroup(prm, kv_heads, 4, 8);
     if (prm.heads_per_wg == 1 && kv_heads > 1 && kv_heads <= 8 && prm.head_tiles == 1) {
         prm.heads_per_wg = kv_heads;
         prm.quarters_per_wg = 1;

@@ -732,6 +732,21 @@ def test_waves_of_large_rows(heads, kv_heads, dim, batch, tokens, waves):
     assert plan["launches"] == 1 and plan["waves_per_workgroup"] == waves
 
 
+@pytest.mark.parametrize("kv_heads,batch,context,expected", [
+    (32, 16, 2048, (8, 4)), (16, 16, 2048, (8, 4)),  # whole rounds of 8-wave workgroups, 1024-token partitions
+    (32, 2, 11032, (4, 2)),                          # 1.4 rounds
+    (16, 4, 4096, (4, 2)), (8, 32, 4096, (4, 1)),    # 512-token partitions; fewer heads (long quarters)
+])
+def test_many_kv_heads_take_wide_workgroups_in_whole_rounds(kv_heads, batch, context, expected):
+    """Waves and KV heads per workgroup of equal-length FP16 calls with D 128 (split 256, 256 CUs)."""
+    lib = cabi.load()
+    width = -(-context // 16)
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_F16, batch, 2 * kv_heads, kv_heads, 128, 16, width,
+                            batch * width, -(-context // 256), 256, cabi.PD_MERGE_SERIAL, cabi.PD_HINT_UNSHARED_PAGES,
+                            np.full(batch, context, dtype=np.int32), 256)
+    assert (plan["waves_per_workgroup"], plan["kv_heads_per_workgroup"]) == expected
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
