@@ -79,7 +79,9 @@ __device__ __forceinline__ void store_empty_states(const PartialParams& p, const
 // a 5-step sum over the lanes for each head and token and a softmax that every
 // lane repeated, and waited for its loads at the end of each block of 32 tokens.
 // A ring of R tiles stays in flight: the next K is requested once a tile is
-// scored, the next V once it is summed. Measured on
+// scored, the next V once it is summed; the range's last ring requests nothing
+// and takes only the tiles that are there (MQA B49 of up to 33 tokens with D 64,
+// us: 9.28 -> 7.88). Measured on
 // MI355X (decode call, us, with the launch shape of plan_fp32; vector ALU ->
 // this): B8 L4096 ragged, 158 MB 44.68 -> 35.66; uniform B2 L4096 23.96 ->
 // 16.11, B16 116.93 -> 101.95;
@@ -295,7 +297,7 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
             load_k(ring[c], at[c]);
             load_v(ring[c], at[c]);
         }
-        for (; s0 < re; s0 += R * TT) {
+        for (; s0 + R * TT < re; s0 += R * TT) {
 #pragma unroll
             for (int c = 0; c < R; ++c) {
                 float x[HG][NL];
@@ -306,6 +308,14 @@ __global__ void __launch_bounds__(kRow ? kWave * fp32_row_max_waves(GT) : kWave 
                 load_v(ring[c], next);
                 at[c] = next;
             }
+        }
+        // The last ring's tiles, as far as the range goes: nothing to request.
+#pragma unroll
+        for (int c = 0; c < R; ++c) {
+            if (s0 + c * TT >= re) break;
+            float x[HG][NL];
+            score(ring[c], x);
+            accumulate(ring[c], at[c], x, s0 + c * TT);
         }
     }
 

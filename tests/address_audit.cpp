@@ -10,7 +10,8 @@
 // stats_offset), following the kernels' loop structure (page-id windows of 64
 // entries, pairs of 16-token tiles for the matrix-core kernel, the next pair
 // requested while one is computed, or the one tile of a short whole-row slice,
-// and rings of kFp32Ring or kFp32RowRing 4-token tiles for the FP32 kernel).
+// and rings of kFp32Ring or kFp32RowRing 4-token tiles for the FP32 kernel; a
+// range's last pair or ring requests nothing).
 // Every global load that its buffer descriptor lets through is
 // checked to lie inside q, k, v, table or lengths, every store inside numerator or stats, every LDS access
 // inside the launch's dynamic LDS; every live token is read from the page its
@@ -320,7 +321,7 @@ void audit_launch(const Problem& pr, const PartialParams& p, bool mfma, Coverage
     if (mfma) AUDIT(mfma_lds_bytes(p, D, pr.kv_elem) <= 160 * 1024, "LDS %d bytes", mfma_lds_bytes(p, D, pr.kv_elem));
     const int align = mfma ? kTileTokens : kFp32TileTokens;
     const int ring = mfma ? 2 : p.row_mode ? kFp32RowRing : kFp32Ring, group_tokens = align;  // tiles in flight per wave
-    const bool last_apart = mfma && last_pair_apart(grid_kind(p), pr.kv_elem);
+    const bool last_apart = !mfma || last_pair_apart(grid_kind(p), pr.kv_elem);
     const int qw = p.quarters_per_wg;
     for (uint32_t bz = 0; bz < grid.z; ++bz) {
         for (uint32_t by = 0; by < grid.y; ++by) {
