@@ -1009,8 +1009,10 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
     // 20.6 against 17.1. The items' waves are not counted: the ragged + shared B16 workload ran 27.2 us per staged call
     // at the 512-token partitions this count picks and 32.5 us at 256 tokens,
     // where counting them against 8 per CU would have stopped.
-    const bool items = prefix_saving(prefix_runs, length_bounds, batch, reach, split_tokens, splits, page_shift,
-                                     slots).saved > 0;
+    auto items = [&] {
+        return prefix_runs != nullptr && prefix_saving(prefix_runs, length_bounds, batch, reach, split_tokens, splits,
+                                                       page_shift, slots).saved > 0;
+    };
     auto enough = [&](int64_t span) {
         int64_t parts = 0, most = 0, fewest = splits;
         for (int b = 0; b < batch; ++b) {
@@ -1020,9 +1022,11 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
             most = live > most ? live : most;
             fewest = lmin(fewest, live);
         }
-        const bool ragged = (!items || span <= kItemSplitTokens) && fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
-        return parts * kQuarters * kv_heads * head_tiles >=
-               static_cast<int64_t>(ragged ? kCoarseWavesRagged : kCoarseWavesPerCu) * cus;
+        const int64_t waves = parts * kQuarters * kv_heads * head_tiles;
+        if (waves >= static_cast<int64_t>(kCoarseWavesPerCu) * cus) return true;
+        const bool ragged = fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
+        return ragged && waves >= static_cast<int64_t>(kCoarseWavesRagged) * cus &&
+               (span <= kItemSplitTokens || !items());
     };
     int c = 1;
     while (2 * c <= splits) {
@@ -1325,10 +1329,14 @@ constexpr int kHalvedListWaves = 14;
 
 inline bool prefers_half_workgroups(const PartialParams& prm, int kv_heads, int cus) {
     if (prm.compact) {
-        const PrefixSaving s = prefix_saving(prm.host_prefix_runs, prm.host_bounds, prm.batch, prm.reach,
-                                             prm.split_tokens, prm.splits, prm.page_shift, prefix_slots(prm.group));
-        return item_workgroups(prm, kv_heads, prm.items - s.saved) * (partial_threads(prm) / kWave) <=
-               static_cast<int64_t>(kHalvedListWaves) * cus;
+        auto fits = [&](int64_t items) {
+            return item_workgroups(prm, kv_heads, items) * (partial_threads(prm) / kWave) <=
+                   static_cast<int64_t>(kHalvedListWaves) * cus;
+        };
+        if (fits(prm.items) || prm.host_prefix_runs == nullptr) return fits(prm.items);
+        return fits(prm.items - prefix_saving(prm.host_prefix_runs, prm.host_bounds, prm.batch, prm.reach,
+                                              prm.split_tokens, prm.splits, prm.page_shift, prefix_slots(prm.group))
+                                    .saved);
     }
     const int64_t whole = shape_workgroups(prm, kv_heads), waves = whole * (partial_threads(prm) / kWave);
     if (waves <= 4ll * cus || waves > 16ll * cus) return false;
