@@ -209,6 +209,30 @@ LARGE = [
 ]
 
 
+# The same bounds with pages of their own, as a cache holds them (fewer sequences of more heads, so the inputs stay small).
+PRIVATE = [(28, 32, 8, 128, 512, 1), (8, 32, 32, 128, 1024, 1), (9, 32, 32, 128, 1024, 2), (14, 64, 16, 64, 1024, 1),
+           (40, 16, 16, 64, 100, 1), (80, 32, 8, 64, 64, 1)]
+
+
+@pytest.mark.parametrize("shape", PRIVATE, ids=lambda s: "x".join(map(str, s[:5])))
+@pytest.mark.parametrize("q_dtype,kv_dtype", FORMATS)
+def test_rows_that_fill_the_device_on_private_pages(shape, q_dtype, kv_dtype):
+    batch, heads, kv_heads, dim, tokens, launches = shape
+    announce(f"whole rows, private pages q={q_dtype} kv={kv_dtype} shape={shape}")
+    width = (tokens + 15) // 16
+    layout = Layout(batch, heads, kv_heads, dim, 16, batch * width)
+    rng = np.random.default_rng(tokens)
+    table = rng.permutation(batch * width).reshape(batch, width).astype(np.int32)
+    lengths = rng.integers(0, tokens + 1, size=batch, dtype=np.int32)
+    lengths[:2] = tokens, 0
+    (q, k, v), (k_scale, v_scale), exact = device_inputs(layout, q_dtype, kv_dtype, seed=batch)
+    plan = DecodePlan(layout, table, lengths, split_tokens=256)
+    if q_dtype != torch.float32 and kv_dtype is None and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert plan.launches(q.dtype) == launches
+    out = plan.run(q, k, v, k_scale=k_scale, v_scale=v_scale).cpu().numpy()
+    assert_parity(out, dense_attention(*exact, table, lengths), bar(q_dtype))
+
+
 @pytest.mark.parametrize("shape", LARGE, ids=lambda s: "x".join(map(str, s[:5])))
 @pytest.mark.parametrize("q_dtype,kv_dtype", FORMATS[1:])
 def test_rows_that_fill_the_device(shape, q_dtype, kv_dtype):
