@@ -91,10 +91,11 @@ enum pd_merge { PD_MERGE_SERIAL = 0, PD_MERGE_SHARED = 1 };
  *   for a batch that does share pages is still correct, only slower. Results
  *   are bit-identical with or without it.
  *   PD_HINT_RAGGED_LENGTHS: the sequence lengths differ widely (live tokens
- *   under about 80% of batch x longest). Grids of up to eight 8-wave
- *   workgroups per CU then run in smaller workgroups, which balance ragged
- *   batches better. Results agree to FP32 rounding (the quarters of a
- *   partition are folded in another grouping); a wrong hint is only slower.
+ *   under about 80% of batch x longest). Larger grids (up to 64 waves per CU
+ *   instead of 16) then stream K and V where nothing is read twice, and the
+ *   four quarters of a long partition are not kept in one workgroup. Results
+ *   agree to FP32 rounding (the quarters of a partition are folded in another
+ *   grouping); a wrong hint is only slower.
  */
 enum pd_hint { PD_HINT_NONE = 0, PD_HINT_UNSHARED_PAGES = 1, PD_HINT_RAGGED_LENGTHS = 2 };
 
@@ -105,7 +106,8 @@ enum pd_hint { PD_HINT_NONE = 0, PD_HINT_UNSHARED_PAGES = 1, PD_HINT_RAGGED_LENG
  * V per (sequence, KV head) -- min(splits * split_tokens, table_width *
  * page_size) tokens -- is instead one whole-row launch (without shared-prefix
  * runs up to 256 KB where the rows come to most of the CUs, and up to 512 KB
- * where they are about one per CU): each workgroup
+ * where they are about one per CU; FP8 rows of several KV heads of 64 dims up to
+ * 160 KB where host bounds are given): each workgroup
  * folds a row's states in LDS and writes out itself, and numerator/stats
  * are left unwritten (they remain required arguments, the workspace of the
  * reference's plan). Results agree with the two-launch path to FP32

@@ -14,11 +14,11 @@
 //     uses them for every query head of the tile (the GQA group, padded to
 //     GT = 1/2/4/8/16 heads), and stores one (m, l, n[D]) state per query head
 //     in slot 4 * partition + quarter of the workspace. A workgroup gathers up
-//     to four KV heads (eight in the FP32 kernel) of the same tokens (their
-//     head slices of a token row are then read together) plus enough quarters
-//     to make four to eight waves, or fewer where such workgroups would
-//     leave most CUs idle. Waves
-//     do not synchronise while they stream; where a workgroup holds several
+//     to four KV heads of the same tokens (their head slices of a token row are
+//     then read together; five or seven where no such divisor fits the 16-bit
+//     kernel) and up to four quarters, eight waves at most and fewer where such
+//     workgroups would leave CUs idle or unevenly loaded. Waves do not
+//     synchronise while they stream; where a workgroup holds several
 //     quarters of one partition (few KV heads), one barrier at the end lets
 //     the first quarter fold the others into a single state. Partitions that
 //     start at or past their sequence's end exit before any load and write
@@ -26,10 +26,10 @@
 //     bounds reach, then a few tail workgroups for lengths that grew past
 //     them on the device.
 //       partial_mfma_kernel (q in FP16 or BF16; K/V in the same type or in
-//       OCP FP8): pairs of 16-token tiles; q.K^T and P.V on the matrix cores, online
-//       softmax with one running max per head and lazy rescaling (the
-//       accumulators are rescaled only when a tile's max exceeds the running
-//       max by 2^8); each lane ends with its own slice of the state and
+//       OCP FP8): pairs of 16-token tiles (one alone for short whole rows); q.K^T
+//       and P.V on the matrix cores, online softmax with one running max per
+//       head and lazy rescaling (the accumulators are rescaled only when a
+//       tile's max exceeds the running max by 2^8); each lane ends with its own slice of the state and
 //       stores it directly.
 //       partial_kernel (FP32): the same decomposition on the FP32 matrix ops;
 //       every row group of lanes keeps its own online-softmax stream, and the

@@ -136,7 +136,7 @@ struct PartialParams {
     int row_allowed;       // the caller takes the output from the partition launch when row_mode is chosen
     int row_mode;          // whole-row workgroups fold every state of a row into out (kFold 2): no merge launch
     int unshared_pages;    // PD_HINT_UNSHARED_PAGES
-    int mid_grid;          // 2-head x 2-quarter workgroups of a mid-size grid
+    int mid_grid;          // a mid-size grid: streams K and V, no fold where the merge is XCD-grouped (plan_mfma)
     int ragged_lengths;    // PD_HINT_RAGGED_LENGTHS
     int stream_mode;       // non-temporal loads: 0 none, 1 V (FP8: K), 2 K and V
     int shape_splits;      // partitions per sequence the bounds reach: the workgroup shape's grid (plan_items)
@@ -1373,21 +1373,20 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     prefer_work_list_for_prefixes(prm, kv_heads, prefix_slots(prm.group), cus);
     // Workgroups of 2 KV heads x 2 quarters (4 waves) where a head's slice of a
     // token row is 256 bytes or more (or there are no more heads), else of 4 KV
-    // heads x 2 quarters (8 waves), where the heads allow it (6 waves for heads of several tiles, three of
-    // which then still take two quarters); a KV head count with no such divisor
-    // keeps its whole token row in one workgroup of one quarter when it fits.
-    // The 16-bit
-    // D 128 kernels need up to 168 VGPRs (three waves per SIMD; their loads
-    // overlap their own computation), so three 4-wave workgroups share a CU,
-    // where an 8-wave workgroup would hold one alone; the others fit 128, and
-    // read half as many bytes of a row per head. Measured on MI355X (decode
-    // call, us, graph; 4 KV heads x 2 quarters in 8 waves / x 1 in 4 / 2 x 2 in
-    // 4): B64 L6144 276.5 / 276.3 / 269.4, B64 L8192 ragged 226.6 / 248.8 /
-    // 226.9, B16 L8192 92.7 / 96.2 / 92.8, page lists loaded on the device (no
-    // bounds) B32 L4096 87.8 / 79.8 / 77.6; FP8 K/V (8 waves / 2 x 2 in 4) B64
-    // L8192 ragged 143.2 / 155.8, B32 L4096 ragged 39.5 / 43.4, B32 L8192 99.3 /
-    // 102.1. B16 ragged with 5 KV heads 28.6 whole, 30.4 as 1 x 4; B8 with 7 KV
-    // heads 25.1 and 26.1.
+    // heads x 2 quarters (8 waves), where the heads allow it (6 waves for heads of
+    // several tiles, three of which then still take two quarters); a KV head count
+    // with no such divisor keeps its whole token row in one workgroup of one
+    // quarter when it fits. The 16-bit D 128 kernels need up to 168 VGPRs (three
+    // waves per SIMD; their loads overlap their own computation), so three 4-wave
+    // workgroups share a CU, where an 8-wave workgroup would hold one alone; the
+    // others fit four or five, and read half as many bytes of a row per head.
+    // Measured on MI355X (decode call, us, graph; 4 KV heads x 2 quarters in 8
+    // waves / x 1 in 4 / 2 x 2 in 4): B64 L6144 276.5 / 276.3 / 269.4, B64 L8192
+    // ragged 226.6 / 248.8 / 226.9, B16 L8192 92.7 / 96.2 / 92.8, page lists loaded
+    // on the device (no bounds) B32 L4096 87.8 / 79.8 / 77.6; FP8 K/V (8 waves / 2 x
+    // 2 in 4) B64 L8192 ragged 143.2 / 155.8, B32 L4096 ragged 39.5 / 43.4, B32 L8192
+    // 99.3 / 102.1. B16 ragged with 5 KV heads 28.6 whole, 30.4 as 1 x 4; B8 with 7
+    // KV heads 25.1 and 26.1.
     const bool wide = head_dim * elem >= 256;
     choose_workgroup(prm, kv_heads, wide ? 2 : 4, !wide && kv_heads > 2 ? 8 : prm.head_tiles > 1 ? 6 : 4);
     const int whole_heads = prm.heads_per_wg;
@@ -1431,7 +1430,7 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     // with), so such launches keep four states per partition.
     //
     // Smaller tiles do fold four quarters where the quarters are long: grids
-    // of more than two 8-wave workgroups per CU over partitions of at least
+    // of more than four waves per CU over partitions of at least
     // 1024 tokens (the coarser partitions of a large grid), with at most 8 KV
     // heads, 16-bit K/V and lengths not flagged ragged, run one KV head x four quarters per
     // 4-wave workgroup (`long_quarters`; the streaming mode stays that of
@@ -1463,11 +1462,19 @@ inline void plan_mfma(PartialParams& prm, int kv_heads, int cus, int head_dim, i
     //     and V streaming is fastest (32K-context MHA at split 256: 92.2; V
     //     only 95.3; neither 98.6). With 25% shared prefix pages (B8 L4096, 32
     //     KV heads): K and V 48.4, V only 43.0.
-    //   - 2 head groups (8 KV heads), no shared pages: V only (B64 L2048
-    //     103.8, K and V 104.7, neither 112.3; a ragged B16 page-32 batch 57.0
-    //     / 62.1 / 64.1). With 25% shared prefix pages (B16 page 32): neither
-    //     50.3, V only 52.0, K and V 59.3.
-    //   - The 2-head x 2-quarter workgroups of mid-size grids: with 2 KV
+    //   - 8 KV heads of 256-byte slices are 4 head groups since workgroups hold
+    //     two heads: no shared pages, K and V / V / neither: B32 L4096 with twice
+    //     the context reserved 90.5 / 94.7 / 104.6, B24 L2048 ragged 30.0 / 29.7 /
+    //     35.3, B16 of 640 tokens 16.0 / 15.3 / 14.9. Pages that may be shared, V /
+    //     neither: B8 L4096 25% shared 23.0 / 24.9, B16 L4096 half shared (a work
+    //     list) 32.5 / 37.6, B40 L2048 ragged 39.0 / 43.6; lists loaded on the
+    //     device (no hint) B16 L3000 32.2 / 39.4, B32 L4096 71.4 / 74.2.
+    //   - 2 head groups of smaller slices (8 KV heads), measured on 4 heads of
+    //     256 bytes, no shared pages: V only (B64 L2048 103.8, K and V 104.7,
+    //     neither 112.3; a ragged B16 page-32 batch 57.0 / 62.1 / 64.1). With 25%
+    //     shared prefix pages (B16 page 32): neither 50.3, V only 52.0, K and V
+    //     59.3; FP8 B40 L2048 ragged with D 64, neither / V (FP8: K): 19.6 / 21.3.
+    //   - Mid-size grids: with 2 KV
     //     heads, one head group, streaming V anyway took B16 L4096 (GQA 8)
     //     from 19.75 to 18.81 us per call. Streaming K as well, on every
     //     mid-size grid with unshared pages, took it to 17.78, and (us per

@@ -1326,7 +1326,7 @@ int main(int argc, char** argv) {
         add(make("edges fp32 page " + std::to_string(page), 8, 8, 2, 64, page, 8,
                  {0, 1, page - 1, page, page + 1, 2 * page - 1, 2 * page + 1, 8 * page}, 1, 4, 4, 7));
     }
-    // Invalid page ids inside live ranges (parked loads) and lengths beyond
+    // Invalid page ids inside live ranges (tiles that read nothing) and lengths beyond
     // the table (clamped).
     {
         Problem pr = make("invalid page ids fp16", 4, 16, 4, 128, 16, 16, {256, 200, 300, 17}, 64, 2, 2, 9);
