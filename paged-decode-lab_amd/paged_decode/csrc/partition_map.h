@@ -983,6 +983,7 @@ inline int prefix_finer_split(int c, const int32_t* runs, const int32_t* bounds,
 // prefix_finer_split may halve c.
 constexpr int64_t kCoarseWaveBytes = 128 * 1024;
 constexpr int kCoarseWavesRagged = 6;
+constexpr double kCoarseFullRagged = 4.1;
 constexpr int kItemSplitTokens = 1024;
 
 struct KernelSplit {
@@ -1006,26 +1007,35 @@ inline KernelSplit coarse_split(int batch, int kv_heads, int head_tiles, int hea
     // tokens FP8 B18 L9434 ragged 44.0 against 58.7, FP16 D 64 B6 L24344 42.6
     // against 52.5; but up to kItemSplitTokens longer partitions are worth more:
     // 16 KV heads B16 L2048, 512 to 1024 tokens, FP8 24.4 against 19.6, FP16 D 64
-    // 20.6 against 17.1. The items' waves are not counted: the ragged + shared B16 workload ran 27.2 us per staged call
-    // at the 512-token partitions this count picks and 32.5 us at 256 tokens,
-    // where counting them against 8 per CU would have stopped.
+    // 20.6 against 17.1. The lower count also takes kCoarseFullRagged waves per CU
+    // of the partitions' tokens (a full partition: four waves per head): contexts
+    // just past a partition leave most of their last one empty (us, against the
+    // coarser split, at 3.0 to 4.0 such waves: GQA 16 B185 of up to 553 tokens 25.3
+    // against 28.6, FP8 B46 of up to 551 17.2 against 18.7, FP8 D 64 B148 L2726 22.8
+    // against 30.6, B43 L1632 a quarter shared 25.0 against 29.3; from 4.16 on FP8 D
+    // 64 B64 L2048 with 4 KV heads 16.2 against 14.6, B32 L4096 27.1 against 25.5).
+    // The items' waves are not counted: the ragged + shared B16 workload ran 27.2 us
+    // per staged call at the 512-token partitions this count picks and 32.5 us at
+    // 256 tokens, where counting them against 8 per CU would have stopped.
     auto items = [&] {
         return prefix_runs != nullptr && prefix_saving(prefix_runs, length_bounds, batch, reach, split_tokens, splits,
                                                        page_shift, slots).saved > 0;
     };
     auto enough = [&](int64_t span) {
-        int64_t parts = 0, most = 0, fewest = splits;
+        int64_t parts = 0, most = 0, fewest = splits, tokens = 0;
         for (int b = 0; b < batch; ++b) {
             const int64_t bound = lmin(reach, length_bounds[b] < 0 ? 0 : length_bounds[b]);
             const int64_t live = (bound + span - 1) / span;
             parts += live;
+            tokens += bound;
             most = live > most ? live : most;
             fewest = lmin(fewest, live);
         }
         const int64_t waves = parts * kQuarters * kv_heads * head_tiles;
         if (waves >= static_cast<int64_t>(kCoarseWavesPerCu) * cus) return true;
         const bool ragged = fewest < most && !(batch <= kCompactMaxBatch && parts * 2 <= batch * most);
-        return ragged && waves >= static_cast<int64_t>(kCoarseWavesRagged) * cus &&
+        const double full = static_cast<double>(tokens) / static_cast<double>(span) * kQuarters * kv_heads * head_tiles;
+        return ragged && waves >= static_cast<int64_t>(kCoarseWavesRagged) * cus && full >= kCoarseFullRagged * cus &&
                (span <= kItemSplitTokens || !items());
     };
     int c = 1;
@@ -1313,18 +1323,19 @@ PD_HD MergeRow merge_xcd_row(uint32_t bx, uint32_t by, int group_rows, int xcd_s
 // halved -- 4 or 8 KV heads to 2 heads x 2 quarters, others to one quarter of
 // their heads: on a rectangular grid when the most loaded CU then holds fewer
 // waves (12 instead of 16 at 12 waves per CU; tail items are not counted; grids of
-// more than 16 are dealt out as CUs get free; up to 4 is a small grid), on a work list, whose items differ, while they leave it at most kHalvedListWaves
-// waves per CU. Measured on MI355X (decode call, us, 8 -> 4 waves): at 12 waves per CU FP8 B6 L4096 16.2 ->
-// 15.5, B24 L2048 ragged 21.4 -> 19.4, B12 L8192 ragged 37.5 -> 32.7, FP16 D 64 B6
-// 15.0 -> 14.0, B12 L8192 ragged 34.8 -> 30.4, 4 KV heads B24 L2048 13.9 -> 12.7;
-// at 6, 8 or 16 FP8 B6 L4096 with 4 KV heads 10.2 -> 10.7, B32 L4096 ragged 35.8 ->
-// 37.0, D 64 with twice the context reserved 25.6 -> 27.4, FP16 D 64 B32 L4096
-// empty to full 30.3 -> 32.6; work lists at 10 to 13 FP8 B32 L4096 half shared
-// 42.6 -> 33.7, a quarter shared 26.2 -> 22.9, FP16 D 64 22.6 -> 20.0, at 15 to 17
-// FP8 D 64 B12 L8192 half shared 20.8 -> 22.9, B64 L2048 14.0 -> 14.4. With 16 KV
-// heads, 4 x 2 -> 4 x 1 (2 x 2): FP8 B6 L4096 ragged 21.0 -> 17.7 (19.3), D 64 with
-// twice the context reserved 19.3 -> 15.4 (18.8), FP16 D 64 22.6 -> 18.8 (20.5);
-// with 3, 3 x 2 -> 3 x 1: FP16 D 64 B32 L3000 ragged 18.6 -> 15.8.
+// more than 16 are dealt out as CUs get free; up to 4 is a small grid), on a work
+// list, whose items differ, while they leave it at most kHalvedListWaves waves per
+// CU. Measured on MI355X (decode call, us, 8 -> 4 waves): at 12 waves per CU FP8
+// B6 L4096 16.2 -> 15.5, B24 L2048 ragged 21.4 -> 19.4, B12 L8192 ragged 37.5 ->
+// 32.7, FP16 D 64 B6 15.0 -> 14.0, B12 L8192 ragged 34.8 -> 30.4, 4 KV heads B24
+// L2048 13.9 -> 12.7; at 6, 8 or 16 FP8 B6 L4096 with 4 KV heads 10.2 -> 10.7, B32
+// L4096 ragged 35.8 -> 37.0, D 64 with twice the context reserved 25.6 -> 27.4,
+// FP16 D 64 B32 L4096 empty to full 30.3 -> 32.6; work lists at 10 to 13 FP8 B32
+// L4096 half shared 42.6 -> 33.7, a quarter shared 26.2 -> 22.9, FP16 D 64 22.6 ->
+// 20.0, at 15 to 17 FP8 D 64 B12 L8192 half shared 20.8 -> 22.9, B64 L2048 14.0 ->
+// 14.4. With 16 KV heads, 4 x 2 -> 4 x 1 (2 x 2): FP8 B6 L4096 ragged 21.0 -> 17.7
+// (19.3), D 64 with twice the context reserved 19.3 -> 15.4 (18.8), FP16 D 64 22.6
+// -> 18.8 (20.5); with 3, 3 x 2 -> 3 x 1: FP16 D 64 B32 L3000 ragged 18.6 -> 15.8.
 constexpr int kHalvedListWaves = 14;
 
 inline bool prefers_half_workgroups(const PartialParams& prm, int kv_heads, int cus) {

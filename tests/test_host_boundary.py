@@ -747,6 +747,19 @@ def test_many_kv_heads_take_wide_workgroups_in_whole_rounds(kv_heads, batch, con
     assert (plan["waves_per_workgroup"], plan["kv_heads_per_workgroup"]) == expected
 
 
+@pytest.mark.parametrize("context,coarse", [(553, False), (1024, True)])
+def test_coarse_split_counts_the_tokens_of_uneven_partitions(context, coarse):
+    """GQA 16, 185 sequences of a quarter of the context to all of it: 512-token partitions that most contexts reach just
+    past, or hardly fill, would leave too little in flight; contexts of two of them do not."""
+    lib = cabi.load()
+    width = -(-context // 16)
+    lengths = np.linspace(context // 4, context, 185).astype(np.int32)
+    plan = cabi.launch_plan(lib, cabi.PD_DTYPE_F16, cabi.PD_DTYPE_F16, 185, 32, 2, 128, 16, width, 185 * width,
+                            -(-context // 256), 256, cabi.PD_MERGE_SERIAL,
+                            cabi.PD_HINT_RAGGED_LENGTHS | cabi.PD_HINT_UNSHARED_PAGES, lengths, 256)
+    assert plan["launches"] == 2 and (plan["kernel_split_tokens"] > 256) == coarse
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
