@@ -1089,7 +1089,10 @@ constexpr int fp32_row_max_waves(int gt) { return gt >= 8 ? 8 : kRowMaxWaves; }
 //     16.9 and 15.5; 1024 tokens ragged 23.8 and 22.7).
 //   - From one row per CU on, 4 waves, so that several workgroups share a CU.
 //   - From four rows per CU on, waves of at least kRowWaveBytes each, but two
-//     of them up to eight rows per CU: the other rows fill the CU.
+//     of them up to eight rows per CU: the other rows fill the CU. FP32 rows of
+//     kRowBytesFp32 keep 4, their waves computing longer per byte (32 / 8 heads, us:
+//     1096 rows of up to 128 tokens with D 64 13.3 -> 12.5, of 64 with D 128 14.1 ->
+//     13.6, 2000 of 103 47.4 -> 45.3; of 42, below, 19.3 -> 21.0).
 // Measured on MI355X (decode call, us, graph; GQA 4, D 128, FP16; as many waves
 // as the LDS holds, up to 12 -> this rule): 2048 rows of up to 256 tokens,
 // ragged, 60.1 -> 36.4 (4 waves; 2: 36.5, 1: 37.6, 8: 54.9), 1024 rows 31.9 ->
@@ -1100,17 +1103,18 @@ constexpr int fp32_row_max_waves(int gt) { return gt >= 8 ? 8 : kRowMaxWaves; }
 // rows 12.4 -> 11.2. MQA rows (16 heads of 64 dims) keep 16 waves: 32 rows of
 // 512 tokens 9.45, 8 waves 9.72.
 constexpr int64_t kRowWaveBytes = 32 * 1024;
+constexpr int64_t kRowBytesFp32 = 64 * 1024;
 constexpr int kRowWavesFew = 8;
 constexpr int kRowWavesMany = 4;
 
-inline int row_waves_for(int64_t rows, int64_t row_bytes, int outputs, int max_waves, int cus) {
+inline int row_waves_for(int64_t rows, int64_t row_bytes, int outputs, int max_waves, int cus, bool fp32) {
     if (rows <= cus) {
         const int one_pass = (outputs + kWave - 1) / kWave;
         if (row_bytes > kRowMaxBytes && one_pass > max_waves) return imin(max_waves, kRowWavesFew);
         return imin(max_waves, imax(kRowWavesFew, one_pass));
     }
     int waves = imin(max_waves, kRowWavesMany);
-    if (rows >= 4ll * cus)
+    if (rows >= 4ll * cus && !(fp32 && row_bytes >= kRowBytesFp32))
         waves = static_cast<int>(lmin(waves, imax(rows >= 8ll * cus ? 1 : 2, static_cast<int>(row_bytes / kRowWaveBytes))));
     return waves;
 }
@@ -1127,7 +1131,8 @@ inline void plan_rows(PartialParams& prm, int kv_heads, int head_dim, int elem, 
                              may_share_prefixes(prm.host_prefix_runs, prm.host_bounds, prm.batch, slots)))
         return;
     const int64_t span = prm.reach;
-    max_waves = row_waves_for(rows, span * head_dim * elem * 2, imin(prm.head_tile, prm.group) * head_dim, max_waves, cus);
+    max_waves = row_waves_for(rows, span * head_dim * elem * 2, imin(prm.head_tile, prm.group) * head_dim, max_waves, cus,
+                              elem == 4);
     int waves = static_cast<int>(lmin(max_waves, (span + kRowWaveTokens - 1) / kRowWaveTokens));
     while (waves > 1 && waves * (slot_bytes + stage_bytes) > 160 * 1024) --waves;
     prm.row_mode = 1;

@@ -760,6 +760,20 @@ def test_coarse_split_counts_the_tokens_of_uneven_partitions(context, coarse):
     assert plan["launches"] == 2 and (plan["kernel_split_tokens"] > 256) == coarse
 
 
+@pytest.mark.parametrize("kv_dtype,dim,batch,tokens,waves", [
+    (cabi.PD_DTYPE_F32, 64, 137, 128, 4), (cabi.PD_DTYPE_F32, 128, 137, 64, 4),  # 64 KB
+    (cabi.PD_DTYPE_F32, 128, 250, 42, 2), (cabi.PD_DTYPE_F16, 64, 137, 128, 2),
+])
+def test_waves_of_many_rows(kv_dtype, dim, batch, tokens, waves):
+    """Whole rows at four to eight per CU (32 / 8 heads, 256 CUs)."""
+    lib = cabi.load()
+    width = -(-tokens // 16)
+    plan = cabi.launch_plan(lib, kv_dtype, kv_dtype, batch, 32, 8, dim, 16, width, batch * width, 1, 256,
+                            cabi.PD_MERGE_SERIAL, cabi.PD_HINT_UNSHARED_PAGES,
+                            np.full(batch, tokens, dtype=np.int32), 256)
+    assert plan["launches"] == 1 and plan["waves_per_workgroup"] == waves
+
+
 def test_launch_planner_invariants_over_random_shapes():
     """The launch planner (`pd_decode_launch_plan`, host only) over 3000 seeded
     random calls: formats, head layouts, pages, table widths up to 4096,
